@@ -203,7 +203,7 @@ def prepare(case, seed):
             s["masks"] = [(np.arange(case["envs"]) % n == k).astype(np.uint8) for k in range(min(n, ACTION_SETS))]
     else:
         # The bodies reach the ground: 2.25 m take 0.7 s of 2 ms steps.
-        for _ in range(350 if case["kind"] == "pile" else 60):
+        for _ in range(350):
             w.step(none, substeps=1)
         s["acts"] = none
     w.synchronize()
