@@ -38,13 +38,16 @@ __device__ __forceinline__ f3 sscale(float s, f3 a) { return {s * a.x, s * a.y, 
 // by its error, would round to either side; to_f32_tie_even settles them. Overflowing quotients
 // land beyond the fp32 range of q and convert to infinity. A zero or infinite divisor keeps the
 // raw reciprocal (+-inf, +-0, exact), so a * y gives the IEEE quotient (+-inf, +-0 or NaN); a
-// NaN divisor gives NaN.
+// NaN divisor gives NaN. For those e is NaN (0 inf), which the minimum replaces by 1/2, and
+// r0 + 3/4 r0 is r0 for r0 = +-inf, +-0; for every other divisor |e| <= 2^-24 and the minimum
+// changes nothing. (A wave issues one VALU instruction per 4 cycles whether or not it depends on
+// the one before, and a compare feeding a select costs 9 more, so the one minimum in place of a
+// class test, a compare and two selects takes 5 instructions off every division group.)
 __device__ __forceinline__ double rcp64(float b) {
     const double d = (double)b;
     const double r0 = __builtin_amdgcn_rcp(d);
-    const double e = __builtin_fma(-d, r0, 1.0);
-    const double r = __builtin_fma(r0, __builtin_fma(e, e, e), r0);
-    return (__builtin_isfinite(b) && b != 0.0f) ? r : r0;
+    const double e = __builtin_fmin(__builtin_fma(-d, r0, 1.0), 0.5);
+    return __builtin_fma(r0, __builtin_fma(e, e, e), r0);
 }
 // fp32(q) for q = fp64(a * y). |q| is first rounded to a multiple of 2^-176 by adding and
 // subtracting C = 1.5 2^-124 (both exact-rounding fp64 operations; -fno-fast-math keeps them):
@@ -72,17 +75,18 @@ __device__ __forceinline__ f3 neg(f3 a) { return {-a.x, -a.y, -a.z}; }
 __device__ __forceinline__ float dot(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ __forceinline__ float len(f3 a) { return __builtin_sqrtf(dot(a, a)); }
 // Square root for a value that is compared against a threshold of at least 2^-47 before the
-// root is used: v_sqrt_f32 followed by the one-ulp correction of a correctly rounded fp32
-// square root (the residuals x - s' s for s' one ulp below and above s decide between the three
-// candidates), without the scaling of inputs below 2^-96 and the final select for 0 and
-// infinity. For x >= 2^-96 the operations are those of the correctly rounded root; +-0, +inf,
-// NaN and negative x come out as the correctly rounded root does (the failing compares keep
-// s); for 0 < x < 2^-96 the result is below 2^-47 and fails every such threshold.
+// root is used: g = v_sqrt_f32(x), within an ulp, plus its residual x - g^2 (exact in an fma)
+// times h, half the reciprocal root from v_rsq_f32. For every x >= 2^-96 this is the correctly
+// rounded root (all of them compared on gfx950), and +-0 gives +-0, NaN and negative normal x NaN.
+// For 0 < x < 2^-96 the result is below 2^-47 and fails every such threshold. 2^-126 keeps the
+// reciprocal root finite at 0 and leaves x >= 2^-96 as it is; at +inf the residual is NaN, which
+// the minimum turns into a number for h = 0 to cancel (residuals of finite x stay below 2^107).
+// 36 cycles against 58 for the two-candidate correction by compares and selects.
 __device__ __forceinline__ float sqrt_gate(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sd = __int_as_float(__float_as_int(s) - 1), su = __int_as_float(__float_as_int(s) + 1);
-    const float t = __builtin_fmaf(-sd, s, x) <= 0.0f ? sd : s;
-    return __builtin_fmaf(-su, s, x) > 0.0f ? su : t;
+    const float g = __builtin_amdgcn_sqrtf(x);
+    const float h = 0.5f * __builtin_amdgcn_rsqf(x + 0x1p-126f);
+    const float d = __builtin_fminf(__builtin_fmaf(-g, g, x), 0x1p120f);
+    return __builtin_fmaf(d, h, g);
 }
 __device__ __forceinline__ float len_gate(f3 a) { return sqrt_gate(dot(a, a)); }
 __device__ __forceinline__ f3 cross(f3 a, f3 b) {
@@ -114,7 +118,18 @@ __device__ __forceinline__ f3 qrot(f3 v, q4 q) {
     return {v.x + 2.0f * (q.w * uv.x + uuv.x), v.y + 2.0f * (q.w * uv.y + uuv.y),
             v.z + 2.0f * (q.w * uv.z + uuv.z)};
 }
-__device__ __forceinline__ float qlen(q4 q) { return __builtin_sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w); }
+// qrot for a vector fixed in a body (an anchor, an axis): the doubling is exact, so the last
+// product and sum are one fma with the same rounding, as long as 2 x does not overflow where
+// v + 2 x would not, i.e. for |v| < 2^103.
+__device__ __forceinline__ f3 qrot_fixed(f3 v, q4 q) {
+    f3 qv = {q.x, q.y, q.z};
+    f3 uv = cross(qv, v);
+    f3 uuv = cross(qv, uv);
+    return {__builtin_fmaf(2.0f, q.w * uv.x + uuv.x, v.x), __builtin_fmaf(2.0f, q.w * uv.y + uuv.y, v.y),
+            __builtin_fmaf(2.0f, q.w * uv.z + uuv.z, v.z)};
+}
+// Only to be compared with 1e-8 and divided by where it is larger (sqrt_gate).
+__device__ __forceinline__ float qlen(q4 q) { return sqrt_gate(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w); }
 __device__ __forceinline__ q4 qnormalize(q4 q) {
     const float l = qlen(q);
     if (!(l > 1e-8f)) return q4{0.0f, 0.0f, 0.0f, 1.0f};
@@ -123,12 +138,25 @@ __device__ __forceinline__ q4 qnormalize(q4 q) {
 // qnormalize with the quotients evaluated before the length test and the identity selected
 // after it (same results; sqrt_gate is exact wherever the test l > 1e-8 passes).
 __device__ __forceinline__ q4 qnormalize_sel(q4 q) {
-    const float l = sqrt_gate(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w);
-    const q4 r = qdivs(q, l);
-    return l > 1e-8f ? r : q4{0.0f, 0.0f, 0.0f, 1.0f};
+    const float l = qlen(q);
+    q4 r = qdivs(q, l);
+    // One scalar branch that is hardly ever taken, in place of a divergent region or four selects.
+    if (__builtin_expect(__ballot(!(l > 1e-8f)) != 0ull, 0)) {
+        if (!(l > 1e-8f)) r = q4{0.0f, 0.0f, 0.0f, 1.0f};
+    }
+    return r;
+}
+// qmul of (d, 0) and q. The terms with the zero scalar part stay (0 b is +-0, or NaN for an
+// infinite b, and decides the sign of a zero sum), each fused with the term after it: 0 b is
+// exact, so the fma rounds what the sum of the two would round.
+__device__ __forceinline__ q4 qmul_vec(f3 d, q4 b) {
+    return {__builtin_fmaf(0.0f, b.x, d.x * b.w) + d.y * b.z - d.z * b.y,
+            __builtin_fmaf(0.0f, b.y, -(d.x * b.z)) + d.y * b.w + d.z * b.x,
+            __builtin_fmaf(0.0f, b.z, d.x * b.y) - d.y * b.x + d.z * b.w,
+            __builtin_fmaf(0.0f, b.w, -(d.x * b.x)) - d.y * b.y - d.z * b.z};
 }
 // Quaternion step q + s * ((d, 0) (x) q) used by every XPBD rotation update.
-__device__ __forceinline__ q4 qdelta(f3 d, q4 q) { return qscale(qmul(mk4(d.x, d.y, d.z, 0.0f), q), 0.5f); }
+__device__ __forceinline__ q4 qdelta(f3 d, q4 q) { return qscale(qmul_vec(d, q), 0.5f); }
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 
 // atan2 / asin after S. Moshier's Cephes single-precision routines (atanf.c, asinf.c):
@@ -166,13 +194,12 @@ __device__ __forceinline__ float z_atan2f(float y, float x) {
     return (__builtin_isnan(x) || __builtin_isnan(y)) ? x + y : res;
 }
 
-__device__ __forceinline__ float z_asinf(float x) {
-    if (__builtin_isnan(x)) return x;
+// For |x| <= 1.
+__device__ __forceinline__ float z_asinf_unit(float x) {
     float a = __builtin_fabsf(x);
-    if (a > 1.0f) return __builtin_nanf("");
     float z, t;
     bool flag = a > 0.5f;
-    if (flag) { z = 0.5f * (1.0f - a); t = __builtin_sqrtf(z); }
+    if (flag) { z = 0.5f * (1.0f - a); t = sqrt_gate(z); }  // z is 0 or at least 2^-25
     else { t = a; z = a * a; }
     float p = ((((4.2163199048e-2f * z + 2.4181311049e-2f) * z + 4.5470025998e-2f) * z + 7.4953002686e-2f) * z + 1.6666752422e-1f) * z * t + t;
     if (flag) p = kPiO2 - (p + p);

@@ -31,15 +31,23 @@ struct EnvLds {
     // u32[hash_keys(G)] (cell << 14 | geom, sorted), then, staged, hpos float4[G] (world
     // centre and radius) and hmeta u32[G] (the model's compact geom word) of each geom.
     uint32_t hkey, hpos;
-    uint32_t bmask;  // contact levels: u64[B][ceil(M/64)] slot masks per body
+    uint32_t bmask;  // contact levels: u64[ceil(M/64)] slot masks per body,
+    uint32_t bmask_stride;  // these many bytes apart
     // Joint solve records with compliance / dt^2 filled in: a per-environment copy used
     // when the model blob is read in place from HBM.
     uint32_t jrec;
     // Candidate-pair broad phase with the model records in HBM: each geom's local centre and
-    // radius (float4[G]) and body | type << 16 (u32[G]), staged once per launch.
-    uint32_t gst, gmeta;
+    // radius (float4[G]) and body | type << 16 (u32[G]), staged once per launch, or (gst_each) on
+    // the pool region before each candidate-pair loop.
+    uint32_t gst, gmeta, gst_each;
     uint32_t obs;                                                      // float[obs']: the observation row
-    uint32_t misc;                                                     // u32[4]: count, pcount, nlev, pad
+    uint32_t misc;                                                     // u32[4]: count, valid slots, nlev, pad
+    uint32_t jw;                                                       // float4[J']: joint contributions (stage C)
+    // Contact pool (make_env_pool): the valid slots alone are in LDS, the list stays in HBM.
+    uint32_t cap;                                                      // slots the pool holds in LDS
+    uint32_t vbod, prv;                                                // u32[cap] each (levels)
+    uint32_t stash;                                                    // uint2[M]: bodies and geoms of each slot
+    uint32_t runs, vmask, wmask;                                       // u64[ceil(M/64)] each
     uint32_t bytes;                                                    // total, multiple of 16
 };
 
@@ -86,6 +94,7 @@ inline EnvLds make_env_lds(uint32_t B, uint32_t Jp, uint32_t N, uint32_t M, uint
     L.skey = take(std::max(std::max(4 * sort_pad(M), 16 * Jp), hash_bytes));  // also stage-C joint contributions, hash
     L.ppen = take(16 * M); L.pimp = take(16 * M);
     L.order = take(2 * sort_pad(M));
+    L.jw = L.skey;
     L.vlist = L.skey; L.lst = L.skey + 2 * M;
     L.loff = L.ppen;  // 16 * M >= 2 * (M + 2) for M >= 1
     L.hkey = L.skey;
@@ -96,6 +105,7 @@ inline EnvLds make_env_lds(uint32_t B, uint32_t Jp, uint32_t N, uint32_t M, uint
     // on the force and torque arrays (dead from integration to the next substep) when they fit.
     const uint32_t mask_words = (M + 63) / 64;
     L.bmask = 8 * mask_words <= 32 ? L.frc : 0u;
+    L.bmask_stride = 8 * mask_words;
     L.jrec = take(jrec_bytes);
     if (8 * mask_words > 32) L.bmask = take(8 * mask_words * B);
     if (stage_geoms) { L.gst = take(16 * G); L.gmeta = take(4 * G); }
@@ -125,7 +135,8 @@ inline EnvLds make_env_lds_small(uint32_t B, uint32_t Jp, uint32_t M, uint32_t G
     const uint32_t hash_bytes = hash_bytes_for(G, true);
     L.con = take(64 * M);
     L.perm = take(2 * M);
-    const uint32_t mask_bytes = masks_in_lds ? 8 * ((M + 63) / 64) * B : 0u;
+    L.bmask_stride = 8 * ((M + 63) / 64);
+    const uint32_t mask_bytes = masks_in_lds ? L.bmask_stride * B : 0u;
     // bmask follows vlist and lst on the sort-key region: the levels run after the sort and
     // the broad phase are done with it.
     const uint32_t lists = align16(std::max(std::max(4 * M + mask_bytes, 4 * sort_pad(M)), 16 * Jp));
@@ -136,12 +147,82 @@ inline EnvLds make_env_lds_small(uint32_t B, uint32_t Jp, uint32_t M, uint32_t G
         L.ppen = take(16 * M); L.pimp = take(16 * M);
     }
     L.order = take(2 * sort_pad(M));
+    L.jw = L.skey;
     L.vlist = L.skey; L.lst = L.skey + 2 * M;
     L.loff = L.ppen;
     L.hkey = L.skey;
     L.hpos = L.skey + (hash ? hash_hpos_off(G) : 0);
     L.bmask = masks_in_lds ? L.skey + 4 * M : kInHbm;
     if (stage_geoms) { L.gst = take(16 * G); L.gmeta = take(4 * G); }
+    L.misc = take(16);
+    L.bytes = o;
+    return L;
+}
+
+// Working sets in LDS without the spatial hash: the contact list stays in HBM and only its
+// valid slots (those the narrow phase finds in contact) are kept in LDS, as pool records of 64 B
+// in slot order:
+//   (point, penetration), (normal, friction), (bias, share a, share b, inverse mass sum),
+//   (bodies a | b << 16, slot, normal impulse, restitution).
+// A step reads of the other slots only their bodies and geoms and writes nothing, so the list
+// has no reason to sit in LDS, where it took three quarters of a robot's working set (64 slots:
+// 6.5 of Ant's 8.5 KB) and so set how many environments a CU holds.
+// `cap` pool records fit in LDS; an environment with more valid slots than that runs its contact
+// solve from its scratch in HBM for that substep.
+//
+// Body records: the float4 of one body side by side, so that one address serves them all and the
+// rest is in the instructions' constant offsets. Split groups: position, orientation, velocity,
+// angular velocity, previous pose, force, torque, velocity at call start (the helper's pose copy
+// and the slot masks use force and torque). Otherwise force and torque, dead from integration on,
+// are on the pool region. Both sizes (36 and 28 words) spread consecutive bodies over the banks.
+//
+// On the pool region, dead until the narrow phase fills it: force, torque and the joint
+// contributions (without split groups), then the staged geoms of the candidate-pair loop, the
+// sort's keys and positions, or the type classes and visiting order of the grouped narrow phase;
+// with the pool in HBM, its slots' bodies and the bodies' last levels. On the level region: with
+// split groups the joint contributions (until integration), then the stash (until the pool is
+// filled), then the levels.
+constexpr uint32_t kPoolMaxList = 1536;  // longer lists keep placement 3 (everything in HBM), as documented
+constexpr uint32_t kPoolFloor = 24;    // smallest pool offered (or the list, or one slot per body)
+constexpr uint32_t kBodyQuadsSplit = 9, kBodyQuads = 7;
+constexpr uint32_t kPoolClasses = 64;  // ordered geom-type pairs of the grouped narrow phase
+inline EnvLds make_env_pool(uint32_t B, uint32_t Jp, uint32_t N, uint32_t M, uint32_t cap, bool split, uint32_t G = 0,
+                            uint32_t jrec_bytes = 0, bool stage_geoms = false, bool sweep = false, uint32_t obsp = 1) {
+    EnvLds L{};
+    uint32_t o = 0;
+    auto take = [&](uint32_t bytes) { uint32_t r = o; o = align16(o + bytes); return r; };
+    const uint32_t body = take(16 * (split ? kBodyQuadsSplit : kBodyQuads) * B);
+    L.pos = body; L.quat = body + 16; L.vel = body + 32; L.angvel = body + 48; L.ppos = body + 64; L.pquat = body + 80;
+    L.vbefore = body + 96;
+    L.jt = take(4 * Jp); L.jp = take(4 * Jp); L.jv = take(4 * Jp);
+    L.lam = take(4 * (N > 0 ? N : 1));
+    L.cap = cap;
+    const uint32_t own = std::max(std::max(64 * cap, 6 * sort_pad(M)), std::max(4 * kPoolClasses + 2 * M, 4 * M + 4 * B));
+    // With the count-only sweep the candidate-pair loop runs only while the list grows, and then
+    // stages its geoms anew; a long list's grouped narrow phase reads their types all the time.
+    L.gst_each = stage_geoms && sweep && M <= 128 ? 1u : 0u;
+    L.con = take(std::max(std::max(own, split ? 0u : 32 * B + 16 * Jp), L.gst_each ? 20 * G : 0u));
+    L.skey = L.con;
+    const uint32_t level = take(std::max(std::max(14 * cap + 4, 8 * M), split ? 16 * Jp : 0u));
+    L.stash = L.vbod = level;
+    L.prv = level + 4 * cap; L.order = level + 8 * cap; L.lst = level + 10 * cap; L.loff = level + 12 * cap;
+    const uint32_t mask_words = (cap + 63) / 64, list_words = (M + 63) / 64;
+    L.bmask_stride = 8 * mask_words;
+    if (split) {
+        L.frc = body + 112; L.trq = body + 128;
+        L.jw = level;
+    } else {
+        L.frc = L.con; L.trq = L.con + 16;  // 32 bytes apart
+        L.jw = L.con + 32 * B;
+    }
+    // Up to four mask words fit a body record's force and torque.
+    if (split && 8 * mask_words <= 32) { L.bmask = L.frc; L.bmask_stride = 16 * kBodyQuadsSplit; }
+    else L.bmask = take(8 * mask_words * B);
+    L.runs = take(8 * list_words); L.vmask = take(8 * list_words); L.wmask = take(8 * list_words);
+    L.jrec = take(jrec_bytes);
+    if (L.gst_each) { L.gst = L.con; L.gmeta = L.con + 16 * G; }
+    else if (stage_geoms) { L.gst = take(16 * G); L.gmeta = take(4 * G); }
+    L.obs = take(4 * obsp);
     L.misc = take(16);
     L.bytes = o;
     return L;
@@ -158,9 +239,10 @@ inline EnvLds make_env_lds_small(uint32_t B, uint32_t Jp, uint32_t M, uint32_t G
 constexpr float kTwoPiF = 6.28318548f;  // 2 * fp32(pi), the largest |2 atan2(y, x)|
 constexpr uint32_t kJRecQuads = 8;  // float4 per solve record
 constexpr uint32_t kJHalfQuads = 4;  // float4 per lane-pair half record
-struct JointPhase { uint32_t type, start, count, pad; };
+struct JointPhase { uint32_t type, start, count, com; };  // com: a body's centre of mass is off its origin
 
-// Record layout (float4 quads). q0 = (ia, ib, template index, flags) [u32]; flags: bit0
+// Record layout (float4 quads). q0 = (ia, ib, template index, flags) [u32], whose x and z the
+// kernel turns into byte offsets in the lane-pair types' halves; flags: bit0
 // inv_m_a > 0, bit1 inv_m_b > 0, bits 8-15 the constraint type.
 // Lane-pair types (POSITIONAL, ANGULAR, ANGULAR_LIMIT) hold two halves, quads 0-3 for the
 // lane of body a and quads 4-7 for the lane of body b, each laid out as
@@ -224,6 +306,12 @@ inline void build_joint_program(const std::vector<ConstraintRec>& tmpl, const st
                             q[6] = make_float4(Bv[0], Bv[1], Bv[2], comp);
                             q[3] = make_float4(com[4 * ia], com[4 * ia + 1], com[4 * ia + 2], 0);
                             q[7] = make_float4(com[4 * ib], com[4 * ib + 1], com[4 * ib + 2], 0);
+                            for (uint32_t x : {ia, ib}) {  // any bit set, a negative zero's included
+                                uint32_t bits[3];
+                                std::memcpy(bits, com + 4 * x, sizeof bits);
+                                const float im = invmi[4 * x];  // light enough to be moved, too heavy to be integrated
+                                if ((bits[0] | bits[1] | bits[2]) != 0u || (im > 0.0f && im < 1e-8f)) ph.com = 1u;
+                            }
                             break;
                         case C_ANGULAR:
                             q[6] = make_float4(Bv[0], Bv[1], Bv[2], comp);
@@ -397,6 +485,12 @@ struct StepArgs {
     // step_subset for envs it did not advance); null when unused.
     const uint8_t* prev_detached;   // [E]
     const ContactRec* prev_contacts; // [E*M]
+    // Contact pool: two scratch lists per environment (the snapshot of a list that this substep
+    // changes, or the levels of a pool too long for LDS; sorted records, or that pool), and the
+    // working list of environments that a step mask holds back.
+    ContactRec* list_snap;          // [E*M]
+    ContactRec* list_tmp;           // [E*M]
+    ContactRec* list_masked;        // [E*M]
     // Optional per-env mask: envs with mask 0 advance only their solver history (lambda,
     // prev contacts, prev count) and keep every visible buffer. Null = all envs.
     const uint8_t* step_mask;       // [E]
@@ -418,7 +512,9 @@ struct StepArgs {
 
 // Where the step kernel keeps the model records and each environment's working set.
 // PL_LDS: both in LDS (several environments per workgroup). PL_MODEL_HBM: the model blob
-// is read in place from HBM (through the caches) and the working set is in LDS.
+// is read in place from HBM (through the caches) and the working set is in LDS. Without the
+// spatial hash these two keep the contact list in HBM and its valid slots in LDS
+// (make_env_pool).
 // PL_ALL_HBM: both in HBM, except the contact pipeline's arrays (make_env_lds_small), which
 // stay in LDS. PL_WORK_HBM: everything in HBM, for contact lists too long for LDS
 // (max_contacts_per_env beyond ~1,400: 64-B records, snapshot and sort keys are ~104 B per

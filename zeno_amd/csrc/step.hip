@@ -37,28 +37,52 @@ __device__ __forceinline__ uint32_t pair_key(uint32_t a, uint32_t b) {
     return (lo << 16) | hi;
 }
 
-struct Lds {
-    float4 *pos, *quat, *vel, *angvel, *ppos, *pquat, *frc, *trq, *vb;
+// Element i of a per-body array whose elements are BS float4 apart: 1 for the separate arrays,
+// more within body records (make_env_pool).
+template <int BS>
+struct BodyArr {
+    float4* p;
+    // A 24-bit product (body indices are 16 bits): one full-rate instruction, where a 32-bit one
+    // takes four times as long.
+    __device__ __forceinline__ float4& operator[](uint32_t i) const {
+        if constexpr (BS == 1) return p[i];
+        else return *(float4*)((unsigned char*)p + __umul24(i, 16u * (uint32_t)BS));
+    }
+    __device__ __forceinline__ BodyArr& operator=(float4* q) { p = q; return *this; }
+};
+
+// BS: float4 per body record; 1, separate arrays.
+template <int BS>
+struct LdsT {
+    BodyArr<BS> pos, quat, vel, angvel, ppos, pquat, vb;
+    BodyArr<BS == (int)kBodyQuads ? 2 : BS> frc, trq;
     float *jt, *jp, *jv, *lam;
     ContactRec* con;
     uint16_t* perm;
     uint32_t* skey;
     float4 *ppen, *pimp;  // prev snapshot: position_pen; impulses.xyz with the pair key in .w
-    float4* jw;  // per-joint force/torque contributions (stage C), aliased on skey
+    float4* jw;  // per-joint force/torque contributions (stage C)
     uint16_t *order, *vlist, *lst, *loff;
     uint32_t* hkey;          // spatial hash, aliased on skey
     float4* hpos;            // spatial hash: geom world centre + radius (then u32 meta[G])
     uint32_t *vbod, *prv;    // contact levels: per-slot dynamic bodies and predecessors (on ppen)
-    unsigned long long* bmask;  // contact levels: per-body slot masks
+    unsigned long long* bmask;  // contact levels: per-body slot masks,
+    uint32_t bmask_stride;      // these many bytes apart
+    __device__ __forceinline__ unsigned long long* mask(uint32_t body) const {
+        return (unsigned long long*)((unsigned char*)bmask + __umul24(body, bmask_stride));
+    }
     float4* jrec;            // per-environment solve records (model records in HBM)
     float4* gst;             // staged geom local centre + radius (model records in HBM, no hash)
     uint32_t* gmeta;         // staged geom body | type << 16
     float* obs;              // the observation row (stage L), written back with the state
+    uint2* stash;            // contact pool: (bodies, geoms) of each slot
+    unsigned long long *runs, *vmask, *wmask;  // contact pool: bits per slot (see list_pass, fill_pool)
     uint32_t* misc;
 };
 
-__device__ __forceinline__ Lds bind_lds(unsigned char* base, const EnvLds& L) {
-    Lds s;
+template <int BS>
+__device__ __forceinline__ LdsT<BS> bind_lds(unsigned char* base, const EnvLds& L) {
+    LdsT<BS> s;
     s.pos = (float4*)(base + L.pos); s.quat = (float4*)(base + L.quat);
     s.vel = (float4*)(base + L.vel); s.angvel = (float4*)(base + L.angvel);
     s.ppos = (float4*)(base + L.ppos); s.pquat = (float4*)(base + L.pquat);
@@ -69,7 +93,7 @@ __device__ __forceinline__ Lds bind_lds(unsigned char* base, const EnvLds& L) {
     s.con = (ContactRec*)(base + L.con);
     s.perm = (uint16_t*)(base + L.perm);
     s.skey = (uint32_t*)(base + L.skey);
-    s.jw = (float4*)(base + L.skey);
+    s.jw = (float4*)(base + L.jw);
     s.ppen = (float4*)(base + L.ppen); s.pimp = (float4*)(base + L.pimp);
     s.order = (uint16_t*)(base + L.order);
     s.vlist = (uint16_t*)(base + L.vlist);
@@ -77,9 +101,14 @@ __device__ __forceinline__ Lds bind_lds(unsigned char* base, const EnvLds& L) {
     s.loff = (uint16_t*)(base + L.loff);
     s.hkey = (uint32_t*)(base + L.hkey);
     s.hpos = (float4*)(base + L.hpos);
-    s.vbod = (uint32_t*)(base + L.ppen + 0u);  // placed by bind_levels
-    s.prv = s.vbod;
+    s.vbod = (uint32_t*)(base + L.vbod);  // contact pool; else placed by bind_levels
+    s.prv = (uint32_t*)(base + L.prv);
+    s.stash = (uint2*)(base + L.stash);
+    s.runs = (unsigned long long*)(base + L.runs);
+    s.vmask = (unsigned long long*)(base + L.vmask);
+    s.wmask = (unsigned long long*)(base + L.wmask);
     s.bmask = (unsigned long long*)(base + L.bmask);
+    s.bmask_stride = L.bmask_stride;
     s.jrec = (float4*)(base + L.jrec);
     s.gst = (float4*)(base + L.gst);
     s.gmeta = (uint32_t*)(base + L.gmeta);
@@ -89,11 +118,11 @@ __device__ __forceinline__ Lds bind_lds(unsigned char* base, const EnvLds& L) {
 }
 
 // Rebinds the arrays of make_env_lds_small to base (working sets in HBM, placement 2).
-__device__ __forceinline__ void bind_small(Lds& s, unsigned char* base, const EnvLds& L) {
+__device__ __forceinline__ void bind_small(LdsT<1>& s, unsigned char* base, const EnvLds& L) {
     s.con = (ContactRec*)(base + L.con);
     s.perm = (uint16_t*)(base + L.perm);
     s.skey = (uint32_t*)(base + L.skey);
-    s.jw = (float4*)(base + L.skey);
+    s.jw = (float4*)(base + L.jw);
     s.ppen = (float4*)(base + L.ppen); s.pimp = (float4*)(base + L.pimp);
     s.order = (uint16_t*)(base + L.order);
     s.vlist = (uint16_t*)(base + L.vlist);
@@ -109,7 +138,7 @@ __device__ __forceinline__ void bind_small(Lds& s, unsigned char* base, const En
 
 // The level computation's per-slot arrays (u32[M] each) at bytes 8M and 12M of the snapshot
 // position array, which is dead once matching is done.
-__device__ __forceinline__ void bind_levels(Lds& s, uint32_t M) {
+__device__ __forceinline__ void bind_levels(LdsT<1>& s, uint32_t M) {
     s.vbod = (uint32_t*)((unsigned char*)s.ppen + 8u * M);
     s.prv = (uint32_t*)((unsigned char*)s.ppen + 12u * M);
 }
@@ -185,7 +214,7 @@ __device__ __forceinline__ void wave_sync() {
 // it could change.
 template <int PERM>
 __device__ __forceinline__ float qperm(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), PERM, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), PERM, 0xF, 0xF, true));
 }
 // quad_perm(1, 0, 3, 2): the partner lane's value.
 __device__ __forceinline__ float pair_swap(float v) { return qperm<0xB1>(v); }
@@ -196,7 +225,7 @@ __device__ __forceinline__ f3 pair_b(f3 v) { return {qperm<0xF5>(v.x), qperm<0xF
 __device__ __forceinline__ q4 pair_a(q4 v) { return {qperm<0xA0>(v.x), qperm<0xA0>(v.y), qperm<0xA0>(v.z), qperm<0xA0>(v.w)}; }
 __device__ __forceinline__ q4 pair_b(q4 v) { return {qperm<0xF5>(v.x), qperm<0xF5>(v.y), qperm<0xF5>(v.z), qperm<0xF5>(v.w)}; }
 // qdelta with its factor 0.5 carrying the lane's sign: sg * (0.5 * x) == (sg * 0.5) * x.
-__device__ __forceinline__ q4 qdelta_signed(f3 d, q4 q, float sg) { return qscale(qmul(mk4(d.x, d.y, d.z, 0.0f), q), 0.5f * sg); }
+__device__ __forceinline__ q4 qdelta_signed(f3 d, q4 q, float sg) { return qscale(qmul_vec(d, q), 0.5f * sg); }
 
 // The lane's half of a lane-pair solve record (build_joint_program): header, the lane's
 // body's inverse mass and inertia, its vector (anchor or axis) with compliance / dt^2 in .w,
@@ -206,9 +235,19 @@ __device__ __forceinline__ JHalf load_half(const float4* p) { return JHalf{p[0],
 // The state a lane-pair solve reads for the lane's body: position, orientation and the
 // constraint's multiplier (every record's header holds a valid multiplier index).
 struct JState { float4 P, Q; float lam; };
-__device__ __forceinline__ JState load_jstate(const JHalf& h, const Lds& s, bool odd) {
-    const uint32_t me = odd ? fbits(h.h0.y) : fbits(h.h0.x);
-    return JState{s.pos[me], s.quat[me], s.lam[fbits(h.h0.z)]};
+// The header's x is the byte offset of the lane's body in the body arrays and its z the
+// multiplier's (fill_alpha).
+template <int BS>
+__device__ __forceinline__ float4* jbody(const BodyArr<BS>& arr, const JHalf& h) {
+    return (float4*)((unsigned char*)arr.p + fbits(h.h0.x));
+}
+template <int BS>
+__device__ __forceinline__ float* jlam(const LdsT<BS>& s, const JHalf& h) {
+    return (float*)((unsigned char*)s.lam + fbits(h.h0.z));
+}
+template <int BS>
+__device__ __forceinline__ JState load_jstate(const JHalf& h, const LdsT<BS>& s) {
+    return JState{*jbody(s.pos, h), *jbody(s.quat, h), *jlam(s, h)};
 }
 
 // Late selects. The positional and hinge solves evaluate their update unconditionally and
@@ -221,11 +260,13 @@ __device__ __forceinline__ JState load_jstate(const JHalf& h, const Lds& s, bool
 // against those thresholds use sqrt_gate, which is the correctly rounded root wherever the
 // comparison can pass.
 
-// :934-1037 positional (point-to-point), lane pair. r - qrot(com, q) is evaluated for every
-// centre of mass: for com = +0 and a finite q the rotated offset is exactly +0 and r - (+0) == r.
-__device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& st, const Lds& s, bool odd) {
-    const uint32_t ia = fbits(h.h0.x), ib = fbits(h.h0.y), ci = fbits(h.h0.z);
-    const uint32_t me = odd ? ib : ia;
+// :934-1037 positional (point-to-point), lane pair. `com`: some body of the phase has its centre
+// of mass off its origin. For com = +0 and a finite q the rotated offset is exactly +0 and
+// r - (+0) == r, and q is finite for every body that the solve moves: integration normalises it,
+// and a normalised quaternion has components within [-1, 1] or is the identity. Phases without
+// such a body, most of every robot's, skip the rotation (33 of about 300 instructions).
+template <int BS>
+__device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd, bool com) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
@@ -233,7 +274,7 @@ __device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& 
     const f3 P = xyz(st.P);
     const q4 Q = toq(st.Q);
     const float lambda_prev = st.lam;
-    const f3 rr = qrot(xyz(h.v1), Q);                      // r_a or r_b
+    const f3 rr = qrot_fixed(xyz(h.v1), Q);                // r_a or r_b
     const f3 u = add(P, rr);                               // pos + r
     const f3 diff = sub(pair_a(u), pair_b(u));             // (pos_a + r_a) - (pos_b + r_b)
     const float C = len_gate(diff);
@@ -243,39 +284,40 @@ __device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& 
     const float w = t + pair_swap(t);                      // (w_a) + (w_b), addition commutes
     const float d_lambda = (-C - alpha_tilde * lambda_prev) / (w + alpha_tilde);
     const f3 impulse = sscale(d_lambda, n);
-    const f3 rc = sub(rr, qrot(xyz(h.v2), Q));
+    f3 rc = rr;
+    if (com) rc = sub(rr, qrot_fixed(xyz(h.v2), Q));
     const f3 Pn = add(P, scale(impulse, sg * inv_mass));
     const q4 Qn = qnormalize_sel(qadd(Q, qdelta_signed(mul(cross(rc, impulse), iI), Q, sg)));
     const bool act = C > 1e-6f, moved = act && inv_mass > 0;
-    s.lam[ci] = act ? lambda_prev + d_lambda : lambda_prev;  // both lanes store the same value
-    set_xyz(&s.pos[me], moved ? Pn : P);
-    s.quat[me] = tof4(moved ? Qn : Q);
+    *jlam(s, h) = act ? lambda_prev + d_lambda : lambda_prev;  // both lanes store the same value
+    set_xyz(jbody(s.pos, h), moved ? Pn : P);
+    *jbody(s.quat, h) = tof4(moved ? Qn : Q);
 }
 
 // :1131-1186 hinge axis alignment, lane pair.
-__device__ __forceinline__ void solve_angular2(const JHalf& h, const JState& st, const Lds& s, bool odd) {
-    const uint32_t me = odd ? fbits(h.h0.y) : fbits(h.h0.x);
+template <int BS>
+__device__ __forceinline__ void solve_angular2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
     const q4 Q = toq(st.Q);
-    const f3 axw = qrot(xyz(h.v1), Q);
+    const f3 axw = qrot_fixed(xyz(h.v1), Q);
     const f3 cr = cross(pair_a(axw), pair_b(axw));
     const float sin_angle = len_gate(cr);
     const f3 n = divs(cr, sin_angle);
-    const float ang_C = z_asinf(clampf(sin_angle, -1.0f, 1.0f));
+    const float ang_C = z_asinf_unit(clampf(sin_angle, -1.0f, 1.0f));  // the clamp also turns NaN into -1
     const float t = dot(mul(n, iI), n);
     const float w = t + pair_swap(t);
     const float d_lambda = -ang_C / (w + alpha_tilde);
     const float dl = odd ? -d_lambda : d_lambda;
     const q4 Qn = qnormalize_sel(qadd(Q, qdelta(mul(sscale(dl, n), iI), Q)));
     const bool moved = sin_angle > 1e-6f && w > 1e-8f && inv_mass > 0;
-    s.quat[me] = tof4(moved ? Qn : Q);
+    *jbody(s.quat, h) = tof4(moved ? Qn : Q);
 }
 
 // :1189-1238 angular limit, lane pair.
-__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JState& st, const Lds& s, bool odd) {
-    const uint32_t me = odd ? fbits(h.h0.y) : fbits(h.h0.x);
+template <int BS>
+__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
@@ -290,7 +332,7 @@ __device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JStat
     if (angle < lower) violation = lower - angle;
     else if (angle > upper) violation = upper - angle;
     if (__builtin_fabsf(violation) > 1e-6f) {
-        const f3 aw = qrot(axis_local, qa);
+        const f3 aw = qrot_fixed(axis_local, qa);
         const float t = dot(mul(aw, iI), aw);
         const float w = t + pair_swap(t);
         // Inside the violation branch (the common case is no violation, which skips the
@@ -298,12 +340,13 @@ __device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JStat
         const float d_lambda = violation / (w + alpha_tilde);
         const f3 ang_impulse = sscale(d_lambda, aw);
         const q4 Qn = qnormalize_sel(qadd(Q, qdelta_signed(mul(ang_impulse, iI), Q, sg)));
-        if (w > 1e-8f && inv_mass > 0) s.quat[me] = tof4(Qn);
+        if (w > 1e-8f && inv_mass > 0) *jbody(s.quat, h) = tof4(Qn);
     }
 }
 
 // :1039-1129 weld (corrects body b only), one lane.
-__device__ __forceinline__ void solve_weld(const float4* r, const Lds& s) {
+template <int BS>
+__device__ __forceinline__ void solve_weld(const float4* r, const LdsT<BS>& s) {
     const float4 q0 = r[0], mb = r[2], a3 = r[3], b4 = r[4], tg = r[5];
     const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
     const float inv_mass_b = mb.x;
@@ -314,7 +357,7 @@ __device__ __forceinline__ void solve_weld(const float4* r, const Lds& s) {
     f3 r_a = qrot(xyz(a3), quat_a);
     f3 r_b = qrot(xyz(b4), quat_b);
     f3 diff = sub(add(pos_a, r_a), add(pos_b, r_b));
-    float C = len(diff);
+    float C = len_gate(diff);  // used only when > 1e-6
     q4 qb = quat_b;
     if (C > 1e-6f) {
         f3 n = divs(diff, C);
@@ -333,7 +376,7 @@ __device__ __forceinline__ void solve_weld(const float4* r, const Lds& s) {
     q4 q_err = qmul(qmul(qconj(qa), qb), qconj(target));
     if (q_err.w < 0) q_err = qneg(q_err);
     f3 e = xyz(q_err);
-    float sh = len(e);
+    float sh = len_gate(e);  // likewise
     if (sh > 1e-6f) {
         f3 axis_rel = divs(e, sh);
         float angle = 2.0f * z_atan2f(sh, q_err.w);
@@ -348,7 +391,8 @@ __device__ __forceinline__ void solve_weld(const float4* r, const Lds& s) {
 }
 
 // :1241-1293 linear limit, one lane.
-__device__ __forceinline__ void solve_linear_limit(const float4* r, const Lds& s) {
+template <int BS>
+__device__ __forceinline__ void solve_linear_limit(const float4* r, const LdsT<BS>& s) {
     const float4 q0 = r[0], ma = r[1], mb = r[2], a3 = r[3], b4 = r[4], lim = r[5];
     const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
     const float inv_mass_a = ma.x, inv_mass_b = mb.x;
@@ -380,7 +424,8 @@ __device__ __forceinline__ void solve_linear_limit(const float4* r, const Lds& s
 }
 
 // :1296-1399 slider, one lane.
-__device__ __forceinline__ void solve_slider(const float4* r, const Lds& s) {
+template <int BS>
+__device__ __forceinline__ void solve_slider(const float4* r, const LdsT<BS>& s) {
     const float4 q0 = r[0], ma = r[1], mb = r[2], a3 = r[3], b4 = r[4], ax = r[5], tg = r[6];
     const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
     const float inv_mass_a = ma.x, inv_mass_b = mb.x;
@@ -394,7 +439,7 @@ __device__ __forceinline__ void solve_slider(const float4* r, const Lds& s) {
     f3 aw = qrot(xyz(ax), quat_a);
     float along = dot(diff, aw);
     f3 perp = sub(diff, sscale(along, aw));
-    float perp_len = len(perp);
+    float perp_len = len_gate(perp);  // used only when > 1e-6
     q4 qa = quat_a, qb = quat_b;
     if (perp_len > 1e-6f) {
         f3 n = divs(perp, perp_len);
@@ -415,7 +460,7 @@ __device__ __forceinline__ void solve_slider(const float4* r, const Lds& s) {
     q4 q_err = qmul(qmul(qconj(qa), qb), qconj(target));
     if (q_err.w < 0) q_err = qneg(q_err);
     f3 e = xyz(q_err);
-    float sh = len(e);
+    float sh = len_gate(e);  // likewise
     if (sh > 1e-6f) {
         f3 axis_err = divs(e, sh);
         float angle_err = 2.0f * z_atan2f(sh, q_err.w);
@@ -466,21 +511,40 @@ struct CRec {
     float rest;          // impulses.w
 };
 
-__device__ __forceinline__ CRec load_crec(const Lds& s, uint32_t phys) {
-    const ContactRec* cr = &s.con[phys];
+// POOL: `slots` is the contact pool (make_env_pool), else the list in the working set.
+template <bool POOL, int BS>
+__device__ __forceinline__ CRec load_crec(const LdsT<BS>& s, float4* slots, uint32_t phys) {
     CRec c;
-    c.pp = *(const float4*)cr->position_pen;
-    c.nf = *(const float4*)cr->normal_friction;
-    c.aux = s.pimp[phys];
-    c.ia = cr->indices[0];
-    c.ib = cr->indices[1];
     c.phys = phys;
-    c.rest = cr->impulses[3];
+    if constexpr (POOL) {
+        const float4* r = slots + 4u * phys;
+        c.pp = r[0];
+        c.nf = r[1];
+        c.aux = r[2];
+        const float4 q = r[3];
+        c.ia = fbits(q.x) & 0xFFFFu;
+        c.ib = fbits(q.x) >> 16;
+        c.rest = q.w;
+    } else {
+        const ContactRec* cr = &s.con[phys];
+        c.pp = *(const float4*)cr->position_pen;
+        c.nf = *(const float4*)cr->normal_friction;
+        c.aux = s.pimp[phys];
+        c.ia = cr->indices[0];
+        c.ib = cr->indices[1];
+        c.rest = cr->impulses[3];
+    }
     return c;
 }
+// The slot's normal impulse.
+template <bool POOL, int BS>
+__device__ __forceinline__ float* slot_impulse(const LdsT<BS>& s, float4* slots, uint32_t phys) {
+    if constexpr (POOL) return (float*)(slots + 4u * phys + 3u) + 2;
+    else return s.con[phys].impulses;
+}
 
-__device__ __forceinline__ void solve_contact_rec(const Mdl& md, const Lds& s, const CRec& c, bool odd) {
-    ContactRec* cr = &s.con[c.phys];
+template <int BS>
+__device__ __forceinline__ void solve_contact_rec(const Mdl& md, const LdsT<BS>& s, const CRec& c, float* jn, bool odd) {
     const float4 pp = c.pp;
     const float4 nf = c.nf;
     const float4 aux = c.aux;
@@ -496,7 +560,7 @@ __device__ __forceinline__ void solve_contact_rec(const Mdl& md, const Lds& s, c
     const float4 P0 = s.pos[me], V0 = s.vel[me], W0 = s.angvel[me];
     // impulses.x (the slot's normal impulse from the previous iteration, written only by
     // this solve) is read with the body state, so that read lands in the same round trip.
-    float jn_prev = cr->impulses[0];
+    float jn_prev = *jn;
     const float sg = odd ? -1.0f : 1.0f;
     const f3 r = sub(cp, xyz(P0));
     const f3 vpt = add(xyz(V0), cross(xyz(W0), r));
@@ -541,11 +605,71 @@ __device__ __forceinline__ void solve_contact_rec(const Mdl& md, const Lds& s, c
         set_xyz(&s.vel[me], v);
         set_xyz(&s.angvel[me], w);
     }
-    cr->impulses[0] = j_n;  // both lanes store the same value
+    *jn = j_n;  // both lanes store the same value
 }
 
-__device__ __forceinline__ void solve_contact2(const Mdl& md, const Lds& s, uint32_t phys, bool odd) {
-    solve_contact_rec(md, s, load_crec(s, phys), odd);
+// Iterations x levels of one substep (S4). Lane pair (2k, 2k+1) takes the k-th slot of each
+// level (and k + G/2, ... when a level holds more). The level lists and the slots' static parts
+// are read ahead over the sequence of (iteration, level) steps: at step f the lane's slot record
+// of step f + 1, its slot index of step f + 2 and the level bounds of step f + 3 are loaded,
+// so a step starts with its record in registers and reads only the bodies' state.
+template <int G, bool POOL, bool HBM, int BS>
+__device__ __forceinline__ void solve_contacts(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, float4* slots, const uint16_t* lst,
+                                               const uint16_t* loff, bool live, int sl, uint32_t max_lev, uint32_t my_nlev) {
+    const bool odd = (sl & 1) != 0;
+    const uint32_t kf = (uint32_t)sl >> 1;
+    const uint32_t nsteps = a.iters * max_lev;
+    // Level bounds of step f: the level's first slot index and its end, read raw (the
+    // lane's slot is first + kf); `ok` when the step exists for the lane's env. The
+    // comparison with the end happens a step later, once the read has landed.
+    auto bounds = [&](uint32_t f, uint32_t lv, uint32_t& first, uint32_t& end) -> bool {
+        first = loff[lv - 1];
+        end = loff[lv];
+        return f < nsteps && live && lv <= my_nlev;
+    };
+    auto next_lv = [&](uint32_t lv) -> uint32_t { return lv == max_lev ? 1u : lv + 1u; };
+    uint32_t j0, e0, j1, e1, j2, e2;
+    uint32_t lv3 = 1;
+    bool v0 = bounds(0, lv3, j0, e0);
+    lv3 = next_lv(lv3);
+    bool v1 = bounds(1, lv3, j1, e1);
+    lv3 = next_lv(lv3);
+    bool v2 = bounds(2, lv3, j2, e2);
+    lv3 = next_lv(lv3);
+    j0 += kf; v0 = v0 && j0 < e0;
+    j1 += kf; v1 = v1 && j1 < e1;
+    CRec cA = load_crec<POOL>(s, slots, v0 ? lst[j0] : 0u), cB;
+    bool cv = v0;
+    uint32_t ce = e0, cj = j0;
+    uint32_t p1 = v1 ? lst[j1] : 0u;
+    // One step with `cur` while the next step's record is loaded into `nxt`; two
+    // steps per trip with the record buffers swapping roles (no record copies).
+    auto cstep = [&](uint32_t f, const CRec& cur, CRec& nxt) {
+        uint32_t j3, e3;
+        const bool ok3 = bounds(f + 3, lv3, j3, e3);
+        lv3 = next_lv(lv3);
+        j2 += kf;
+        v2 = v2 && j2 < e2;
+        const uint32_t p2 = v2 ? lst[j2] : 0u;
+        nxt = load_crec<POOL>(s, slots, p1);
+        if (cv) {
+            solve_contact_rec(md, s, cur, slot_impulse<POOL>(s, slots, cur.phys), odd);
+            for (uint32_t j = cj + G / 2; j < ce; j += G / 2) {
+                const uint32_t phys = lst[j];
+                solve_contact_rec(md, s, load_crec<POOL>(s, slots, phys), slot_impulse<POOL>(s, slots, phys), odd);
+            }
+        }
+        wave_sync<HBM>();
+        cv = v1; ce = e1; cj = j1;
+        p1 = p2; v1 = v2; e1 = e2; j1 = j2;
+        v2 = ok3; e2 = e3; j2 = j3;
+    };
+    uint32_t f = 0;
+    for (; f + 2 <= nsteps; f += 2) {
+        cstep(f, cA, cB);
+        cstep(f + 1, cB, cA);
+    }
+    if (f < nsteps) cstep(f, cA, cB);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -553,16 +677,18 @@ __device__ __forceinline__ void solve_contact2(const Mdl& md, const Lds& s, uint
 // ---------------------------------------------------------------------------------------
 // AHEAD (model records in HBM): both geom records are read whole at the start, so their reads
 // are in flight together instead of some waiting behind the type tests.
-template <bool AHEAD>
-__device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, const Lds& s, ContactRec* c) {
-    const uint32_t body_a = c->indices[0], body_b = c->indices[1];
+struct NarrowHit { f3 normal, cp; float pen, mu; bool hit; };
+
+template <bool AHEAD, int BS>
+__device__ __forceinline__ NarrowHit narrow_eval(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, uint32_t body_a, uint32_t body_b,
+                                                 uint32_t geom_a, uint32_t geom_b) {
     GeomRec la, lb;
     if constexpr (AHEAD) {
-        la = md.geoms[c->indices[2]];
-        lb = md.geoms[c->indices[3]];
+        la = md.geoms[geom_a];
+        lb = md.geoms[geom_b];
     }
-    const GeomRec& ga = AHEAD ? la : md.geoms[c->indices[2]];
-    const GeomRec& gb = AHEAD ? lb : md.geoms[c->indices[3]];
+    const GeomRec& ga = AHEAD ? la : md.geoms[geom_a];
+    const GeomRec& gb = AHEAD ? lb : md.geoms[geom_b];
     const f3 pos_a = add(xyz(s.pos[body_a]), mk3(ga.pos_size0[0], ga.pos_size0[1], ga.pos_size0[2]));
     const f3 pos_b = add(xyz(s.pos[body_b]), mk3(gb.pos_size0[0], gb.pos_size0[1], gb.pos_size0[2]));
     const uint32_t type_a = ga.type_body[0], type_b = gb.type_body[0];
@@ -572,7 +698,7 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
     if (type_a == GEOM_SPHERE && type_b == GEOM_SPHERE) {
         float ra = ga.pos_size0[3], rb = gb.pos_size0[3];
         f3 diff = sub(pos_b, pos_a);
-        float dist = len(diff);
+        float dist = len_gate(diff);
         float min_dist = ra + rb;
         if (dist < min_dist && dist > 1e-6f) {
             normal = divs(diff, dist);
@@ -631,10 +757,15 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
             hit = true;
         }
     }
-    if (hit) {
-        float mu = __builtin_sqrtf(ga.params[2] * gb.params[2]);
-        *(float4*)c->position_pen = make_float4(cp.x, cp.y, cp.z, pen);
-        *(float4*)c->normal_friction = make_float4(normal.x, normal.y, normal.z, mu);
+    return NarrowHit{normal, cp, pen, hit ? __builtin_sqrtf(ga.params[2] * gb.params[2]) : 0.0f, hit};
+}
+
+template <bool AHEAD, int BS>
+__device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, ContactRec* c) {
+    const NarrowHit h = narrow_eval<AHEAD>(a, md, s, c->indices[0], c->indices[1], c->indices[2], c->indices[3]);
+    if (h.hit) {
+        *(float4*)c->position_pen = make_float4(h.cp.x, h.cp.y, h.cp.z, h.pen);
+        *(float4*)c->normal_friction = make_float4(h.normal.x, h.normal.y, h.normal.z, h.mu);
         *(float4*)c->impulses = make_float4(0.0f, 0.0f, 0.0f, a.restitution);
     } else {
         c->position_pen[3] = -1.0f;
@@ -644,10 +775,11 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
 // One joint solve of the given type on the lane pair: h is the lane's half record and st its
 // body's state (lane-pair types), r the whole record in LDS (single-lane types, run by body
 // a's lane, which read the state themselves).
-__device__ __forceinline__ void solve_joint(uint32_t type, const JHalf& h, const JState& st, const float4* r, const Lds& s,
-                                            bool odd) {
+template <int BS>
+__device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const JState& st, const float4* r,
+                                            const LdsT<BS>& s, bool odd) {
     switch (type) {
-        case C_POSITIONAL: solve_positional2(h, st, s, odd); break;
+        case C_POSITIONAL: solve_positional2(h, st, s, odd, com); break;
         case C_ANGULAR: solve_angular2(h, st, s, odd); break;
         case C_ANGULAR_LIMIT: solve_angular_limit2(h, st, s, odd); break;
         case C_WELD: if (!odd) solve_weld(r, s); break;
@@ -719,8 +851,8 @@ __device__ __forceinline__ void sort_keys_1024(uint32_t* key, uint32_t n, uint32
 // pair k to logical slot `slot + k` while that is below M.
 // STAGED: the geom data come from hpos / hmeta (working sets in HBM); otherwise from the
 // model records and the body poses directly (both in LDS, or the model records in cache).
-template <bool STAGED>
-__device__ __forceinline__ float4 hash_geom_pos(const Mdl& md, const Lds& s, uint32_t g) {
+template <bool STAGED, int BS>
+__device__ __forceinline__ float4 hash_geom_pos(const Mdl& md, const LdsT<BS>& s, uint32_t g) {
     if (STAGED) return s.hpos[g];
     const GeomRec& gr = md.geoms[g];
     return tof4(add(xyz(s.pos[gr.type_body[1]]), mk3(gr.pos_size0[0], gr.pos_size0[1], gr.pos_size0[2])), gr.pos_size0[3]);
@@ -749,8 +881,8 @@ __device__ __forceinline__ bool hash_filter_pass(const StepArgs& a, const Mdl& m
     return ((fa.x & gr.type_body[2]) | (gr.type_body[3] & fa.y)) != 0u;
 }
 
-template <bool STAGED>
-__device__ __forceinline__ uint32_t hash_pairs_of(const StepArgs& a, const Mdl& md, const Lds& s, const uint32_t* hmeta, uint32_t g, bool emit,
+template <bool STAGED, int BS>
+__device__ __forceinline__ uint32_t hash_pairs_of(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, const uint32_t* hmeta, uint32_t g, bool emit,
                                   uint32_t slot) {
     const float4 pa4 = hash_geom_pos<STAGED>(md, s, g);
     const uint32_t wa = hash_geom_meta<STAGED>(md, hmeta, g);
@@ -838,8 +970,8 @@ __device__ __forceinline__ uint32_t hash_pairs_of(const StepArgs& a, const Mdl& 
 // each lane walks its own candidates, or, when one lane holds more than twice the mean, the
 // wave's candidates are dealt out four per lane at a time, each lane finding its candidate's
 // run by a search over the lanes' prefix sums, so a crowded cell does not hold the wave up.
-template <bool STAGED>
-__device__ __forceinline__ uint32_t hash_count_forward(const StepArgs& a, const Mdl& md, const Lds& s, const uint32_t* hmeta, int lane) {
+template <bool STAGED, int BS>
+__device__ __forceinline__ uint32_t hash_count_forward(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, const uint32_t* hmeta, int lane) {
     constexpr int R = 5;
     const uint32_t NG = a.G;
     uint32_t hits = 0;
@@ -1035,6 +1167,240 @@ __device__ __forceinline__ uint32_t hash_count_forward(const StepArgs& a, const 
     return hits;
 }
 
+// ---------------------------------------------------------------------------------------
+// Contact pool (make_env_pool): the contact list stays in HBM, in the state's own array, and
+// each substep keeps only its valid slots in LDS.
+// ---------------------------------------------------------------------------------------
+// Level arrays of a pool that does not fit in LDS, in the environment's snapshot scratch (dead
+// once the matching is done): 14 M + 4 of its 64 M bytes. The pool itself is then in the other
+// scratch list.
+struct SpillArrays { uint32_t *vbod, *cnt; uint16_t *order, *lst, *loff; };
+__device__ __forceinline__ SpillArrays spill_arrays(ContactRec* scratch, uint32_t M) {
+    unsigned char* const b = (unsigned char*)scratch;
+    return SpillArrays{(uint32_t*)b, (uint32_t*)(b + 4 * (size_t)M), (uint16_t*)(b + 8 * (size_t)M), (uint16_t*)(b + 10 * (size_t)M),
+                       (uint16_t*)(b + 12 * (size_t)M)};
+}
+
+__device__ __forceinline__ void copy_record(ContactRec* to, const ContactRec* from) {
+    const float4* f = (const float4*)from;
+    const float4 q0 = f[0], q1 = f[1], q2 = f[2], q3 = f[3];
+    float4* t = (float4*)to;
+    t[0] = q0; t[1] = q1; t[2] = q2; t[3] = q3;
+}
+
+// sort_contacts (:711-745) on the list in HBM: the stable order of the first n slots by pair key,
+// then the records that change places move through `tmp`. Keys (and, for lists longer than
+// kMaxRecsPerLane slots per lane, the bitonic network's positions) are on the pool region.
+template <int G, int BS>
+__device__ __forceinline__ void sort_list(const LdsT<BS>& s, ContactRec* list, ContactRec* tmp, bool need, uint32_t n, int sl) {
+    const bool big = __ballot(need && n > (uint32_t)(kMaxRecsPerLane * G)) != 0ull;
+    if (!big) {
+        if (need) {
+            for (uint32_t k = sl; k < n; k += G) {
+                const uint2 ib = *(const uint2*)list[k].indices;
+                s.skey[k] = pair_key(ib.x, ib.y);
+            }
+        }
+        wave_sync<false>();
+        uint32_t dst[kMaxRecsPerLane];
+        if (need) {
+#pragma unroll
+            for (int r = 0; r < kMaxRecsPerLane; ++r) {
+                const uint32_t k = sl + r * G;
+                dst[r] = k;
+                if (k < n) {
+                    const uint32_t key = s.skey[k];
+                    uint32_t rank = 0;
+                    for (uint32_t j = 0; j < n; ++j) {
+                        const uint32_t kj = s.skey[j];
+                        rank += (kj < key || (kj == key && j < k)) ? 1u : 0u;
+                    }
+                    dst[r] = rank;
+                    if (rank != k) copy_record(&tmp[rank], &list[k]);
+                }
+            }
+        }
+        wave_sync<true>();
+        if (need) {
+#pragma unroll
+            for (int r = 0; r < kMaxRecsPerLane; ++r) {
+                const uint32_t k = sl + r * G;
+                if (k < n && dst[r] != k) copy_record(&list[k], &tmp[k]);
+            }
+        }
+    } else {
+        // The network runs to the wave's largest padded length.
+        uint32_t np = 1;
+        while (np < n) np <<= 1;
+        uint32_t wave_np = need ? np : 1u;
+        for (uint32_t d = 1; d < 64u; d <<= 1) {
+            const uint32_t t = __shfl_xor(wave_np, d);
+            wave_np = t > wave_np ? t : wave_np;
+        }
+        uint32_t* const key = s.skey;
+        if (need) {
+            for (uint32_t k = sl; k < np; k += G) {
+                uint32_t v = 0xFFFFFFFFu;
+                if (k < n) {
+                    const uint2 ib = *(const uint2*)list[k].indices;
+                    v = pair_key(ib.x, ib.y);
+                }
+                key[k] = v;
+            }
+        }
+        uint16_t* const place = (uint16_t*)(key + np);  // 6 np bytes in all
+        if (need) {
+            for (uint32_t k = sl; k < np; k += G) place[k] = (uint16_t)k;
+        }
+        wave_sync<false>();
+        for (uint32_t kk = 2; kk <= wave_np; kk <<= 1) {
+            for (uint32_t j = kk >> 1; j > 0; j >>= 1) {
+                if (need && kk <= np) {
+                    for (uint32_t t = sl; t < np / 2; t += G) {
+                        const uint32_t i = ((t & ~(j - 1u)) << 1) | (t & (j - 1u));
+                        const uint32_t l = i | j;
+                        const uint32_t xa = key[i], xb = key[l];
+                        const uint32_t ia = place[i], ib = place[l];
+                        const bool gt = xa > xb || (xa == xb && ia > ib);
+                        if (gt == ((i & kk) == 0)) {
+                            key[i] = xb; key[l] = xa;
+                            place[i] = (uint16_t)ib; place[l] = (uint16_t)ia;
+                        }
+                    }
+                }
+                wave_sync<false>();
+            }
+        }
+        if (need) {
+            for (uint32_t k = sl; k < n; k += G) {
+                if (place[k] != k) copy_record(&tmp[k], &list[place[k]]);
+            }
+        }
+        wave_sync<true>();
+        if (need) {
+            for (uint32_t k = sl; k < n; k += G) {
+                if (place[k] != k) copy_record(&list[k], &tmp[k]);
+            }
+        }
+    }
+    wave_sync<true>();
+}
+
+// match_cached_contacts (:1483-1544) and the solve's constants for every pool slot: the bias
+// velocity, the two position-correction shares and the summed inverse mass, the same in every
+// iteration. The snapshot entries with the slot's body pair form one run (it is key-sorted), whose
+// starts are the bits of s.runs; the match is the run's first entry at the smallest squared
+// distance below 0.04 (the reference's first strict minimum in index order), read four entries a
+// trip. Also sets the slot's dynamic bodies in vbod and, with bmask, their slot masks.
+// Returns whether some slot of this lane writes both of its bodies.
+template <int G, int BS>
+__device__ __forceinline__ bool match_pool(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, float4* pool, uint32_t* vbod, bool masks,
+                                           const ContactRec* snap, uint32_t pn, bool same, uint32_t nv, int sl) {
+    bool two_bodies = false;
+    auto key_of = [&](uint32_t i) {
+        const uint2 ib = *(const uint2*)snap[i].indices;
+        return pair_key(ib.x, ib.y);
+    };
+    for (uint32_t i = sl; i < nv; i += G) {
+        float4* const rec = pool + 4u * i;
+        const float4 pp = rec[0], q = rec[3];
+        const uint32_t ia = fbits(q.x) & 0xFFFFu, ib = fbits(q.x) >> 16, k = fbits(q.y);
+        const float4 ma = md.invmi[ia], mb = md.invmi[ib];
+        const uint32_t fa = md.flags[ia], fb = md.flags[ib];
+        const uint32_t key = pair_key(ia, ib);
+        uint32_t lo, end = 0;
+        bool found;
+        if (k < pn && (same || key_of(k) == key)) {
+            // The run holding entry k: the highest run start at or below it.
+            uint32_t w = k >> 6;
+            unsigned long long m = s.runs[w] & (~0ull >> (63u - (k & 63u)));
+            while (m == 0ull) m = s.runs[--w];  // entry 0 starts a run
+            lo = w * 64u + 63u - (uint32_t)__clzll(m);
+            found = true;
+        } else {
+            uint32_t hi = pn;
+            lo = 0;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (key_of(mid) < key) lo = mid + 1; else hi = mid;
+            }
+            found = lo < pn && key_of(lo) == key;
+        }
+        float jn = 0.0f;
+        if (found) {
+            // The run ends at the next run start.
+            uint32_t w = lo >> 6;
+            unsigned long long m = (lo & 63u) == 63u ? 0ull : s.runs[w] & (~0ull << ((lo & 63u) + 1u));
+            while (m == 0ull && (w + 1u) * 64u < pn) m = s.runs[++w];
+            end = m != 0ull ? w * 64u + (uint32_t)__ffsll(m) - 1u : pn;
+            float best = 0.04f;
+            const f3 p = xyz(pp);
+            auto visit = [&](bool in, float4 e, float imp) {
+                if (!in || e.w < 0) return;
+                const f3 d = sub(xyz(e), p);
+                const float dsq = dot(d, d);
+                if (dsq < best) { best = dsq; jn = imp * 0.8f; }
+            };
+            for (uint32_t j = lo; j < end; j += 4) {
+                const uint32_t j1 = j + 1 < end ? j + 1 : j, j2 = j + 2 < end ? j + 2 : j, j3 = j + 3 < end ? j + 3 : j;
+                const float4 e0 = *(const float4*)snap[j].position_pen, e1 = *(const float4*)snap[j1].position_pen;
+                const float4 e2 = *(const float4*)snap[j2].position_pen, e3 = *(const float4*)snap[j3].position_pen;
+                const float i0 = snap[j].impulses[0], i1 = snap[j1].impulses[0], i2 = snap[j2].impulses[0], i3 = snap[j3].impulses[0];
+                visit(true, e0, i0);
+                visit(j + 1 < end, e1, i1);
+                visit(j + 2 < end, e2, i2);
+                visit(j + 3 < end, e3, i3);
+            }
+        }
+        const float inv_mass_sum = ma.x + mb.x;
+        const float pos_correction = a.baumgarte * fmaxf(pp.w - a.slop, 0.0f);
+        const float bias = pos_correction / a.dt;
+        rec[2] = make_float4(bias, pos_correction * (ma.x / inv_mass_sum), pos_correction * (mb.x / inv_mass_sum), inv_mass_sum);
+        *((float2*)(rec + 3) + 1) = make_float2(jn, a.restitution);
+        const uint32_t A = (fa & 2u) ? ia : 0xFFFFu, Bd = (fb & 2u) ? ib : 0xFFFFu;
+        vbod[i] = A | (Bd << 16);
+        if (masks) {
+            const unsigned long long bit = 1ull << (i & 63u);
+            if (A != 0xFFFFu) atomicOr(s.mask(A) + (i >> 6), bit);
+            if (Bd != 0xFFFFu) atomicOr(s.mask(Bd) + (i >> 6), bit);
+        }
+        two_bodies = two_bodies || (A != 0xFFFFu && Bd != 0xFFFFu);
+    }
+    return two_bodies;
+}
+
+// Contact levels of a pool in HBM, by one lane per environment in slot order (level = 1 + the
+// larger of the two bodies' last levels); last(b) is body b's, zero. Returns the number of levels.
+template <class F>
+__device__ __forceinline__ uint32_t spill_levels(const SpillArrays& sp, const F& last, uint32_t nv) {
+    uint32_t nlev = 0;
+    for (uint32_t i = 0; i < nv; ++i) {
+        const uint32_t bo = sp.vbod[i], A = bo & 0xFFFFu, Bd = bo >> 16;
+        const uint32_t la = A != 0xFFFFu ? last(A) : 0u, lb = Bd != 0xFFFFu ? last(Bd) : 0u;
+        const uint32_t lv = (la > lb ? la : lb) + 1u;
+        if (A != 0xFFFFu) last(A) = lv;
+        if (Bd != 0xFFFFu) last(Bd) = lv;
+        sp.order[i] = (uint16_t)lv;
+        nlev = lv > nlev ? lv : nlev;
+    }
+    for (uint32_t l = 0; l < nlev; ++l) sp.cnt[l] = 0u;
+    for (uint32_t i = 0; i < nv; ++i) { const uint32_t l = sp.order[i] - 1u; sp.cnt[l] = sp.cnt[l] + 1u; }
+    uint32_t run = 0;
+    sp.loff[0] = 0;
+    for (uint32_t l = 0; l < nlev; ++l) {
+        const uint32_t c = sp.cnt[l];
+        sp.cnt[l] = run;
+        run += c;
+        sp.loff[l + 1] = (uint16_t)run;
+    }
+    for (uint32_t i = 0; i < nv; ++i) {
+        const uint32_t l = sp.order[i] - 1u, at = sp.cnt[l];
+        sp.lst[at] = (uint16_t)i;
+        sp.cnt[l] = at + 1u;
+    }
+    return nlev;
+}
+
 // PL: where the model records and the working sets live (Placement): PL_LDS, both in LDS
 // (EPW environments per wave, and up to kMaxWaves independent waves per workgroup sharing one
 // copy of the model records); PL_MODEL_HBM, the model blob read in place from HBM and one
@@ -1068,6 +1434,8 @@ void step_kernel(StepArgs a) {
     // Placement 2 with the spatial hash keeps the previous-contact snapshot on the hash's
     // arrays (make_env_lds_small): it is taken after the broad phase.
     constexpr bool LATE_SNAP = HASH && PL == PL_ALL_HBM;
+    // Working sets in LDS, no spatial hash: the contact list in HBM, its valid slots in a pool.
+    constexpr bool POOL = !HASH && !HBM;
     static_assert(PL == PL_LDS || EPW == 1, "model records in HBM run one environment per workgroup");
     static_assert(!HASH || EPW == 1, "the spatial hash runs one environment per workgroup");
     static_assert(!GROUP || EPW == 1, "type-grouped narrow phase: one environment per workgroup");
@@ -1075,7 +1443,9 @@ void step_kernel(StepArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = (int)(threadIdx.x & (kWave - 1));    // lane
     constexpr bool MULTI = PL == PL_LDS && !HASH;          // several waves per workgroup possible
-    const uint32_t wv = MULTI ? threadIdx.x / kWave : 0u;  // wave in this workgroup
+    // Wave in this workgroup, the same in every lane (so the addresses that follow from it and the
+    // branches between a group's two waves are scalar).
+    const uint32_t wv = MULTI ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0u;
     const uint32_t W = MULTI ? blockDim.x / kWave : 1u;    // waves in this workgroup
     const uint32_t NG = SPLIT ? W / 2u : W;                 // environment groups in this workgroup
     const bool helper = SPLIT && wv >= NG;                  // split: the group's second wave
@@ -1088,13 +1458,15 @@ void step_kernel(StepArgs a) {
     const bool live = env < a.E;
     unsigned char* const env_base = HBM ? a.work + (size_t)wave_id * a.lds.bytes
                                         : smem + (PL == PL_LDS ? a.ml.bytes : 0u) + grp * EPW * a.lds.bytes;
-    Lds s = bind_lds(env_base + le * a.lds.bytes, a.lds);
+    constexpr int BS = !POOL ? 1 : SPLIT ? (int)kBodyQuadsSplit : (int)kBodyQuads;
+    using Lds = LdsT<BS>;
+    Lds s = bind_lds<BS>(env_base + le * a.lds.bytes, a.lds);
     // The HBM working set's own snapshot arrays, unused by placement 2 but for a substep whose
     // appends may wrap the count past 2^32 (LATE_SNAP below).
     float4* const hppen = s.ppen;
     float4* const hpimp = s.pimp;
-    if (PL == PL_ALL_HBM) bind_small(s, smem, a.lds_small);  // PL_WORK_HBM: all of it in a.work
-    bind_levels(s, a.M);
+    if constexpr (PL == PL_ALL_HBM) bind_small(s, smem, a.lds_small);  // PL_WORK_HBM: all of it in a.work
+    if constexpr (!POOL) bind_levels(s, a.M);
     Mdl md = bind_model(PL == PL_LDS ? smem : (const unsigned char*)a.model, a.ml);
     if (PL != PL_LDS) md.jrec = s.jrec;
     const uint32_t B = a.B, M = a.M, N = a.N, Jp = a.Jp;
@@ -1179,6 +1551,12 @@ void step_kernel(StepArgs a) {
     // into LDS: the contact records are most of the bytes, and the helper needs them only after
     // integration, while the solver's body reads then meet no contact traffic.
     auto load_contacts = [&]() {
+        if constexpr (POOL) {
+            count = a.counts[env];
+            pcount = a.pcounts[env];
+            detached = a.prev_detached != nullptr && a.prev_detached[env] != 0;
+            return;
+        }
         if (sl < M) c0 = read_slot(&gc[sl]);
         if (sl + G < M) c1 = read_slot(&gc[sl + G]);
         if (sl + 2 * G < M) c2 = read_slot(&gc[sl + 2 * G]);
@@ -1188,6 +1566,20 @@ void step_kernel(StepArgs a) {
         detached = a.prev_detached != nullptr && a.prev_detached[env] != 0;
     };
     if (!SPLIT && live) load_contacts();
+    auto stage_geoms = [&]() {
+        // Two geoms per lane and trip, both read before either is written.
+        for (uint32_t g = tid; g < a.G; g += 2u * kWave) {
+            const uint32_t g2 = g + kWave;
+            const float4 ps = *(const float4*)md.geoms[g].pos_size0;
+            const uint4 tb = *(const uint4*)md.geoms[g].type_body;
+            float4 ps2 = ps;
+            uint4 tb2 = tb;
+            if (g2 < a.G) { ps2 = *(const float4*)md.geoms[g2].pos_size0; tb2 = *(const uint4*)md.geoms[g2].type_body; }
+            s.gst[g] = ps;
+            s.gmeta[g] = tb.y | (tb.x << 16);
+            if (g2 < a.G) { s.gst[g2] = ps2; s.gmeta[g2] = tb2.y | (tb2.x << 16); }
+        }
+    };
     // With the model records in HBM, the working-set reads follow the copy of the solve
     // records and the geom staging without a barrier in between, so their HBM latencies
     // overlap.
@@ -1212,20 +1604,7 @@ void step_kernel(StepArgs a) {
     } else if (PL != PL_LDS) {
         const uint4* src = a.model + a.ml.jrec / 16u;
         for (uint32_t i = tid; i < a.nrec * kJRecQuads; i += kWave) ((uint4*)s.jrec)[i] = src[i];
-        if (!HASH) {
-            // Two geoms per lane and trip, both read before either is written.
-            for (uint32_t g = tid; g < a.G; g += 2u * kWave) {
-                const uint32_t g2 = g + kWave;
-                const float4 ps = *(const float4*)md.geoms[g].pos_size0;
-                const uint4 tb = *(const uint4*)md.geoms[g].type_body;
-                float4 ps2 = ps;
-                uint4 tb2 = tb;
-                if (g2 < a.G) { ps2 = *(const float4*)md.geoms[g2].pos_size0; tb2 = *(const uint4*)md.geoms[g2].type_body; }
-                s.gst[g] = ps;
-                s.gmeta[g] = tb.y | (tb.x << 16);
-                if (g2 < a.G) { s.gst[g2] = ps2; s.gmeta[g2] = tb2.y | (tb2.x << 16); }
-            }
-        }
+        if (!HASH && !a.lds.gst_each) stage_geoms();
     }
 
     // alpha~ = compliance / dt^2 (all_shaders.metal:928), the same value for every solve of
@@ -1236,6 +1615,11 @@ void step_kernel(StepArgs a) {
             if (joint_type_paired((fbits(q[0].w) >> 8) & 0xFFu)) {
                 q[2].w = q[2].w / (a.dt * a.dt);
                 q[6].w = q[6].w / (a.dt * a.dt);
+                // Each half's header: its own body and the multiplier, as byte offsets.
+                q[0].x = __uint_as_float(fbits(q[0].x) * (16u * (uint32_t)BS));
+                q[4].x = __uint_as_float(fbits(q[4].y) * (16u * (uint32_t)BS));
+                q[0].z = __uint_as_float(fbits(q[0].z) * 4u);
+                q[4].z = __uint_as_float(fbits(q[4].z) * 4u);
             } else {
                 q[3].w = q[3].w / (a.dt * a.dt);
             }
@@ -1286,12 +1670,48 @@ void step_kernel(StepArgs a) {
             s.perm[k] = (uint16_t)k;
         }
     };
-    if (!SPLIT && live) write_contacts();
+    if (!POOL && live) write_contacts();
     __syncthreads();  // below, each wave syncs with itself (split groups: three barriers per substep)
     if (PL != PL_LDS) fill_alpha(tid, kWave);
+    // Contact pool: the list the substeps work on (the state's own; for an environment that a step
+    // mask holds back, a copy, as its visible list stays) and the environment's scratch lists.
+    ContactRec* list = nullptr;
+    ContactRec *slist = nullptr, *tlist = nullptr;
+    constexpr int CH = 64 / G;  // chunks of G slots in a 64-slot word of the masks
+    if constexpr (POOL) {
+        // Lanes past the last environment point at its lists, which they may read ahead but not use.
+        const size_t first = (size_t)(live ? env : a.E - 1u) * M;
+        list = (stepped || !live ? a.contacts : a.list_masked) + first;
+        slist = a.list_snap + first;
+        tlist = a.list_tmp + first;
+        if (do_prep) {
+            if (SPLIT && live) load_contacts();
+            if (live && !stepped) {
+                for (uint32_t k = sl; k < M; k += G) copy_record(&list[k], &gc[k]);
+            }
+            wave_sync<true>();
+        }
+    }
+    const uint64_t group_mask = (G == 64) ? ~0ull : (((1ull << (G % 64)) - 1ull) << (le * G));
+    const uint64_t below = (sl == 0) ? 0ull : ((~0ull) >> (64 - sl)) << (le * G);
+    // The environment's lanes' bits of a wave mask.
+    auto group_bits = [&](uint64_t b) -> uint64_t { return G == 64 ? b : (b >> (le * G)) & ((1ull << (G % 64)) - 1ull); };
     tick(PH_LOAD);
 
+    const int lane_of_env = sl;
+    const Lds launch_s = s;
     for (uint32_t step = 0; step < a.substeps; ++step) {
+        // Opaque in each substep, so that the addresses that follow from the lane are formed where
+        // they are used: hoisted out of this loop they are some fifty registers, which the compiler
+        // spills to scratch.
+        int sl = lane_of_env;
+        asm volatile("" : "+v"(sl));
+        Lds s = launch_s;
+        if constexpr (POOL && EPW > 1) {
+            uint32_t at = le * a.lds.bytes;
+            asm volatile("" : "+v"(at));
+            s = bind_lds<BS>(env_base + at, a.lds);
+        }
         // ---- Previous-contact snapshot (cache_contacts of the last substep) -----------
         // A split group's helper takes it after the first barrier of the substep (with the
         // contact list's LDS copy in the first substep), so the solver never waits for it.
@@ -1313,8 +1733,44 @@ void step_kernel(StepArgs a) {
                                       __uint_as_float(pair_key(r->indices[0], r->indices[1])));
             }
         };
+        // Contact pool. A full list that this substep cannot wrap takes no append and keeps its
+        // order, so it is its own snapshot: nothing of it changes before the matching is done. Any
+        // other list is copied first. The first 64 slots' bodies and geoms, which need no pose, are
+        // read here, so that they land while the forces and the integration run.
+        bool full = false, same = false;  // same: the snapshot is the list, entry for entry
+        const ContactRec* snap = list;
+        uint32_t pn = 0;
+        uint4 ix[CH];
+        float ipen[CH];
+        auto read_word = [&](const ContactRec* from, uint32_t lim, uint32_t base) {
+#pragma unroll
+            for (int r = 0; r < CH; ++r) {
+                const uint32_t i = base + (uint32_t)(r * G + sl);
+                ix[r] = make_uint4(0, 0, 0, 0);
+                ipen[r] = -1.0f;
+                if (i < lim) { ix[r] = *(const uint4*)from[i].indices; ipen[r] = from[i].position_pen[3]; }
+            }
+        };
+        if constexpr (POOL) {
+            if (do_prep) {
+                if (step > 0) wave_sync<true>();  // the last substep's writes to the list
+                pn = live ? (pcount < M ? pcount : M) : 0u;
+                full = live && count >= M && count <= 0xFFFFFFFFu - a.P && !(a.sort_all != 0u && step == 0);
+                const bool det = step == 0 && detached;
+                same = full && !det && pn == M;
+                snap = det ? a.prev_contacts + (size_t)env * M : full ? list : slist;
+                const bool keep = live && !full && !det;
+                if (__ballot(keep) != 0ull) {
+                    if (keep) {
+                        for (uint32_t k = sl; k < pn; k += G) copy_record(&slist[k], &list[k]);
+                    }
+                    wave_sync<true>();
+                }
+                read_word(snap, pn, 0);
+            }
+        }
         const bool snap_first = LATE_SNAP && (uint64_t)count + (uint64_t)a.G * (uint64_t)(a.G - 1u) / 2u > 0xFFFFFFFFull;
-        if (!SPLIT && (!LATE_SNAP || snap_first) && live) snapshot(M, snap_first ? hppen : s.ppen, snap_first ? hpimp : s.pimp);
+        if (!POOL && (!LATE_SNAP || snap_first) && live) snapshot(M, snap_first ? hppen : s.ppen, snap_first ? hpimp : s.pimp);
         // Stage B (below), one text for the two places it runs from.
         const bool take_vb = alias && step == 0;  // aliased: the velocity at call start
         auto stage_b = [&]() {
@@ -1545,19 +2001,6 @@ void step_kernel(StepArgs a) {
         tick(PH_FORCES);
         if (SPLIT) {
             __syncthreads();  // split barrier 1: poses after integration are in place
-            if (live && helper) {
-                if (step == 0) {
-                    count = a.counts[env];
-                    pcount = a.pcounts[env];
-                    detached = a.prev_detached != nullptr && a.prev_detached[env] != 0;
-#pragma unroll 4
-                    for (uint32_t k = sl; k < M; k += G) {
-                        write_slot(&s.con[k], read_slot(&gc[k]));
-                        s.perm[k] = (uint16_t)k;
-                    }
-                }
-                snapshot(M, s.ppen, s.pimp);
-            }
         }
         // ---- E: broad_phase (S1), :468-533, or the spatial hash, :556-703 -------------
         // Broad phase to contact levels: the helper's part of a split group, on the poses
@@ -1565,9 +2008,34 @@ void step_kernel(StepArgs a) {
         // them after the narrow phase).
         if (do_prep) {
         Lds sp = s;
-        if (SPLIT) { sp.pos = s.frc; sp.quat = s.trq; }
+        if constexpr (SPLIT) { sp.pos = s.frc; sp.quat = s.trq; }
         Lds& s = sp;
         const uint32_t count_before = count;
+        if constexpr (POOL) {
+            // One pass over the snapshot: s.runs, the starts of its runs of one body pair. Where the
+            // snapshot is the list, also the list's bodies and geoms (s.stash) and s.wmask, the
+            // slots whose record does not say "no contact" yet.
+            uint32_t carry = 0;
+            for (uint32_t base = 0; base < M; base += 64) {
+                if (base > 0) read_word(snap, pn, base);
+                uint64_t starts = 0, touched = 0;
+#pragma unroll
+                for (int r = 0; r < CH; ++r) {
+                    const uint32_t i = base + (uint32_t)(r * G + sl);
+                    const uint32_t key = pair_key(ix[r].x, ix[r].y);
+                    uint32_t prev = __shfl_up(key, 1, G);
+                    if (sl == 0) prev = carry;
+                    carry = __shfl(key, G - 1, G);
+                    starts |= group_bits(__ballot(i < pn && (i == 0u || key != prev))) << (r * G);
+                    touched |= group_bits(__ballot(fbits(ipen[r]) != fbits(-1.0f))) << (r * G);
+                    if (same && i < M) s.stash[i] = make_uint2(ix[r].x | (ix[r].y << 16), ix[r].z | (ix[r].w << 16));
+                }
+                if (live && sl == 0) {
+                    s.runs[base >> 6] = starts;
+                    if (same) s.wmask[base >> 6] = touched;
+                }
+            }
+        }
         if (HASH) {
             uint32_t* const hmeta = (uint32_t*)(s.hpos + a.G);
             // Cells (broad_phase_count_cells, :556-584), sort keys and each geom's staged
@@ -1684,8 +2152,6 @@ void step_kernel(StepArgs a) {
             for (uint32_t d = 1; d < 64u; d <<= 1) hits += (uint32_t)__shfl_xor((int)hits, (int)d);
             count += a.sweep_planes + hits;
         } else {
-            const uint64_t group_mask = (G == 64) ? ~0ull : (((1ull << (G % 64)) - 1ull) << (le * G));
-            const uint64_t below = (sl == 0) ? 0ull : ((~0ull) >> (64 - sl)) << (le * G);
             // With the model records in HBM the geoms come from their LDS copy (s.gst /
             // s.gmeta) and the loop is software-pipelined over chunks of G pairs: while chunk
             // k is tested, the pair list of chunk k + 2 (HBM) and the staged geoms of chunk
@@ -1694,6 +2160,7 @@ void step_kernel(StepArgs a) {
             auto pair_at = [&](uint32_t p) -> uint32_t { return (live && p < a.P) ? md.pairs[p] : 0u; };
             uint32_t pr1 = 0, pr2 = 0, m1a = 0, m1b = 0;
             float4 c1a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), c1b = c1a;
+            if (GSTAGE && !HASH && a.lds.gst_each) { stage_geoms(); wave_sync<HBM>(); }
             if (GSTAGE && a.P > 0) {
                 pr1 = pair_at(sl);
                 pr2 = pair_at(sl + G);
@@ -1750,8 +2217,12 @@ void step_kernel(StepArgs a) {
                 if (hit) {
                     const uint32_t slot = count + rank;
                     if (slot < M) {
-                        uint32_t* idx = s.con[s.perm[slot]].indices;
-                        idx[0] = ba; idx[1] = bb; idx[2] = g; idx[3] = h;
+                        if constexpr (POOL) {
+                            *(uint4*)list[slot].indices = make_uint4(ba, bb, g, h);
+                        } else {
+                            uint32_t* idx = s.con[s.perm[slot]].indices;
+                            idx[0] = ba; idx[1] = bb; idx[2] = g; idx[3] = h;
+                        }
                     }
                 }
                 count += total;
@@ -1774,6 +2245,12 @@ void step_kernel(StepArgs a) {
             const bool wrote = (a.sort_all != 0u && step == 0) ||
                                (count != count_before && (count_before < M || count < count_before));
             const bool need = live && wrote && n > 1;
+            if constexpr (POOL) {
+                if (__ballot(live && !full) != 0ull) {
+                    wave_sync<true>();  // the appended slots' bodies and geoms
+                    if (__ballot(need) != 0ull) sort_list<G>(s, list, tlist, need, n, sl);
+                }
+            } else {
             const bool big = __ballot(need && n > (uint32_t)(kMaxRecsPerLane * G)) != 0ull;
             if (!big) {
                 if (need) {
@@ -1858,11 +2335,151 @@ void step_kernel(StepArgs a) {
                     for (uint32_t k = sl; k < n; k += G) s.perm[k] = s.order[k];
                 }
             }
+            }
         }
         wave_sync<HBM>();
         tick(PH_BROAD);
         // ---- F: narrow_phase (:751-894) -----------------------------------------------
         const uint32_t n_live = count < M ? count : M;
+        uint32_t nv = 0;           // valid slots
+        bool two_bodies = false;   // some valid slot of this lane writes both of its bodies
+        bool spill = false;        // the wave's pools are in the scratch lists
+        const uint32_t mw = ((POOL ? a.lds.cap : M) + 63u) >> 6;  // mask words per body
+        if constexpr (POOL) {
+            if (__ballot(live && !same) != 0ull) {
+                for (uint32_t base = 0; base < M; base += 64) {
+                    read_word(list, live && !same ? n_live : 0u, base);
+                    uint64_t touched = 0;
+#pragma unroll
+                    for (int r = 0; r < CH; ++r) {
+                        const uint32_t i = base + (uint32_t)(r * G + sl);
+                        touched |= group_bits(__ballot(fbits(ipen[r]) != fbits(-1.0f))) << (r * G);
+                        if (live && !same && i < n_live)
+                            s.stash[i] = make_uint2(ix[r].x | (ix[r].y << 16), ix[r].z | (ix[r].w << 16));
+                    }
+                    if (live && !same && sl == 0) s.wmask[base >> 6] = touched;
+                }
+            }
+            wave_sync<false>();
+            const uint32_t cap = a.lds.cap;
+            float4* const pool = (float4*)s.con;
+            // Appends the wave's valid slots k (one per lane) to their environments' pools, in slot
+            // order, and returns the environment's bits.
+            auto put = [&](bool hit, uint32_t k, uint2 st, float4 q0, float4 q1) -> uint64_t {
+                const uint64_t ballot = __ballot(hit);
+                if (hit) {
+                    const uint32_t at = nv + (uint32_t)__popcll(ballot & below);
+                    const float4 q3 = make_float4(__uint_as_float(st.x), __uint_as_float(k), 0.0f, 0.0f);
+                    if (at < cap) { pool[4 * at] = q0; pool[4 * at + 1] = q1; pool[4 * at + 3] = q3; }
+                    else { float4* const t = (float4*)&tlist[at]; t[0] = q0; t[1] = q1; t[3] = q3; }
+                }
+                nv += (uint32_t)__popcll(ballot & group_mask);
+                return group_bits(ballot);
+            };
+            auto eval = [&](uint2 st) { return narrow_eval<PL != PL_LDS>(a, md, s, st.x & 0xFFFFu, st.x >> 16, st.y & 0xFFFFu, st.y >> 16); };
+            if (GROUP && a.ext_contacts && M >= 64) {
+                // Extended mode: each slot's pair type picks one of detectCollision's branches,
+                // and a wave runs every branch that its lanes need. The slots are visited grouped
+                // by (type a, type b), a counting sort over the 64 ordered type pairs on the pool
+                // region; the results wait in the scratch list, and a second pass in slot order
+                // fills the pool. Each slot's result depends on that slot alone, so the visiting
+                // order changes no result.
+                uint32_t* const ccount = (uint32_t*)s.con;
+                uint16_t* const visit = (uint16_t*)(ccount + kPoolClasses);
+                auto geom_type = [&](uint32_t g) -> uint32_t { return PL != PL_LDS && !a.lds.gst_each ? s.gmeta[g] >> 16 : md.geoms[g].type_body[0]; };
+                auto slot_class = [&](uint2 st) -> uint32_t {
+                    return (geom_type(st.y & 0xFFFFu) & 7u) * 8u + (geom_type(st.y >> 16) & 7u);
+                };
+                static_assert(!GROUP || G == 64, "one class per lane");
+                ccount[sl] = 0u;
+                for (uint32_t w = sl; w < (M + 63u) / 64u; w += G) s.vmask[w] = 0ull;
+                wave_sync<false>();
+                if (live) {
+                    for (uint32_t k = sl; k < n_live; k += G) atomicAdd(&ccount[slot_class(s.stash[k])], 1u);
+                }
+                wave_sync<false>();
+                const uint32_t sum = ccount[sl];
+                uint32_t incl = sum;
+                for (int d = 1; d < G; d <<= 1) {
+                    const uint32_t t = __shfl_up(incl, d, G);
+                    if (sl >= d) incl += t;
+                }
+                ccount[sl] = incl - sum;
+                wave_sync<false>();
+                if (live) {
+                    for (uint32_t k = sl; k < n_live; k += G) visit[atomicAdd(&ccount[slot_class(s.stash[k])], 1u)] = (uint16_t)k;
+                }
+                wave_sync<false>();
+                if (live) {
+                    for (uint32_t i = sl; i < n_live; i += G) {
+                        const uint32_t k = visit[i];
+                        const NarrowHit h = eval(s.stash[k]);
+                        if (!h.hit) continue;
+                        float4* const t = (float4*)&tlist[k];
+                        t[0] = tof4(h.cp, h.pen);
+                        t[1] = tof4(h.normal, h.mu);
+                        atomicOr(&s.vmask[k >> 6], 1ull << (k & 63u));
+                    }
+                }
+                wave_sync<true>();
+                for (uint32_t base = 0; base < M; base += G) {
+                    const uint32_t k = base + (uint32_t)sl;
+                    const bool hit = live && k < n_live && ((s.vmask[k >> 6] >> (k & 63u)) & 1ull) != 0ull;
+                    float4 q0 = make_float4(0, 0, 0, 0), q1 = q0;
+                    uint2 st = make_uint2(0, 0);
+                    if (hit) { const float4* t = (const float4*)&tlist[k]; q0 = t[0]; q1 = t[1]; st = s.stash[k]; }
+                    put(hit, k, st, q0, q1);  // at most slot k of the scratch list is written: k and below are read
+                }
+            } else {
+                for (uint32_t base = 0; base < M; base += 64) {
+                    uint64_t valid = 0;
+                    for (uint32_t r = 0; r < (uint32_t)CH && base + r * G < M; ++r) {
+                        const uint32_t k = base + r * G + (uint32_t)sl;
+                        NarrowHit h{};
+                        uint2 st = make_uint2(0, 0);
+                        if (live && k < n_live) { st = s.stash[k]; h = eval(st); }
+                        valid |= put(h.hit, k, st, tof4(h.cp, h.pen), tof4(h.normal, h.mu)) << (r * G);
+                    }
+                    if (live && sl == 0) s.vmask[base >> 6] = valid;
+                }
+            }
+            spill = __ballot(live && nv > cap) != 0ull;
+            wave_sync<false>();
+            // ---- G: match_cached_contacts, the solve's constants and the slot masks ----------
+            if (!spill) {
+                if (live) {
+                    for (uint32_t b = sl; b < B; b += G) {
+                        for (uint32_t w = 0; w < mw; ++w) s.mask(b)[w] = 0ull;
+                    }
+                }
+                wave_sync<false>();
+                if (live) two_bodies = match_pool<G>(a, md, s, pool, s.vbod, true, snap, pn, same, nv, sl);
+            } else {
+                auto last = [&](uint32_t b) -> uint32_t& { return ((uint32_t*)s.con)[M + b]; };  // behind `bodies` below
+                const SpillArrays sa = spill_arrays(slist, M);
+                if (live) {
+                    for (uint32_t i = sl; i < (nv < cap ? nv : cap); i += G) copy_record(&tlist[i], (const ContactRec*)&pool[4 * i]);
+                }
+                wave_sync<true>();
+                if (live) {
+                    for (uint32_t i = sl; i < B; i += G) last(i) = 0u;
+                }
+                // The level arrays overlay the snapshot scratch, so vbod waits in the pool's LDS
+                // (its records are in the scratch now) until the snapshot is done with.
+                uint32_t nlev = 0;
+                uint32_t* const bodies = (uint32_t*)s.con;
+                if (live) (void)match_pool<G>(a, md, s, (float4*)tlist, bodies, false, snap, pn, same, nv, sl);
+                wave_sync<true>();
+                if (live) {
+                    for (uint32_t i = sl; i < nv; i += G) sa.vbod[i] = bodies[i];
+                }
+                wave_sync<true>();
+                if (live && sl == 0) nlev = spill_levels(sa, last, nv);
+                if (live && sl == 0) s.misc[2] = nlev;
+                wave_sync<true>();
+            }
+            if (live && sl == 0) s.misc[1] = nv;
+        } else {
         if (GROUP && a.ext_contacts && M >= 64) {
             // Extended mode: each slot's pair type picks one of detectCollision's branches,
             // and a wave runs every branch that its lanes need. The slots are visited grouped
@@ -1986,6 +2603,7 @@ void step_kernel(StepArgs a) {
                 }
             }
         }
+        }  // POOL
         // ---- Contact levels for S4 -----------------------------------------------------
         // level(slot) = 1 + max level of earlier valid slots sharing a body that the solve
         // writes (inv_m > 1e-8). Running levels in order reproduces the sequential slot
@@ -2000,17 +2618,13 @@ void step_kernel(StepArgs a) {
         // slots are then placed by a counting sort into s.lst, level l owning
         // [s.loff[l - 1], s.loff[l]).
         wave_sync<HBM>();  // matching has read the snapshot, which the level arrays reuse
-        uint32_t nv = 0;
-        const uint32_t mw = (M + 63u) >> 6;                                        // mask words per body
         uint32_t* const vbod = s.vbod;  // u32[M] dynamic bodies
         uint32_t* const prv = s.prv;    // u32[M] predecessors, then the level counters
-        const uint64_t group_mask = (G == 64) ? ~0ull : (((1ull << (G % 64)) - 1ull) << (le * G));
-        const uint64_t below = (sl == 0) ? 0ull : ((~0ull) >> (64 - sl)) << (le * G);
+        if constexpr (!POOL) {
         if (live) {
             for (uint32_t i = sl; i < B * mw; i += G) s.bmask[i] = 0ull;
         }
         wave_sync<HBM>();
-        bool two_bodies = false;  // some valid slot of this lane writes both of its bodies
         if (live) {
             for (uint32_t base = 0; base < n_live; base += G) {
                 const uint32_t k = base + sl;
@@ -2029,13 +2643,15 @@ void step_kernel(StepArgs a) {
                     s.vlist[at] = (uint16_t)phys;
                     vbod[at] = A | (Bd << 16);
                     const unsigned long long bit = 1ull << (at & 63u);
-                    if (A != 0xFFFFu) atomicOr(&s.bmask[A * mw + (at >> 6)], bit);
-                    if (Bd != 0xFFFFu) atomicOr(&s.bmask[Bd * mw + (at >> 6)], bit);
+                    if (A != 0xFFFFu) atomicOr(s.mask(A) + (at >> 6), bit);
+                    if (Bd != 0xFFFFu) atomicOr(s.mask(Bd) + (at >> 6), bit);
                     two_bodies = two_bodies || (A != 0xFFFFu && Bd != 0xFFFFu);
                 }
                 nv += (uint32_t)__popcll(ballot & group_mask);
             }
         }
+        }  // !POOL
+        if (!spill) {
         const bool relax = (__ballot(two_bodies) & group_mask) != 0ull;  // per environment
         wave_sync<HBM>();
         if (live && !relax) {
@@ -2044,7 +2660,7 @@ void step_kernel(StepArgs a) {
                 const uint32_t body = (bo & 0xFFFFu) != 0xFFFFu ? (bo & 0xFFFFu) : (bo >> 16);
                 uint32_t lv = 1;
                 if (body != 0xFFFFu) {
-                    const unsigned long long* m = &s.bmask[body * mw];
+                    const unsigned long long* m = s.mask(body);
                     for (uint32_t w = 0; w < (i >> 6); ++w) lv += (uint32_t)__popcll(m[w]);
                     lv += (uint32_t)__popcll(m[i >> 6] & ((1ull << (i & 63u)) - 1ull));
                 }
@@ -2055,7 +2671,7 @@ void step_kernel(StepArgs a) {
         auto pred = [&](uint32_t body, uint32_t i) -> uint32_t {
             if (body == 0xFFFFu) return 0xFFFFu;
             for (int w = (int)(i >> 6); w >= 0; --w) {
-                unsigned long long m = s.bmask[body * mw + (uint32_t)w];
+                unsigned long long m = s.mask(body)[w];
                 if ((uint32_t)w == (i >> 6)) m &= (1ull << (i & 63u)) - 1ull;
                 if (m) return (uint32_t)w * 64u + 63u - (uint32_t)__clzll(m);
             }
@@ -2133,13 +2749,14 @@ void step_kernel(StepArgs a) {
             }
             wave_sync<HBM>();
             if (live) {
-                for (uint32_t i = sl; i < nv; i += G) s.lst[atomicAdd(&cnt[s.order[i] - 1u], 1u)] = s.vlist[i];
+                for (uint32_t i = sl; i < nv; i += G) s.lst[atomicAdd(&cnt[s.order[i] - 1u], 1u)] = POOL ? (uint16_t)i : s.vlist[i];
             }
         }
+        }  // !spill
         // Per-slot constants of the contact solve (the same in every iteration): the bias
         // velocity, the two position-correction shares and the summed inverse mass, kept in
-        // the snapshot's impulse array, which is dead once matching is done.
-        if (live) {
+        // the snapshot's impulse array, which is dead once matching is done (the pool's: match_pool).
+        if (!POOL && live) {
             for (uint32_t i = sl; i < nv; i += G) {
                 const uint32_t phys = s.vlist[i];
                 const ContactRec* c = &s.con[phys];
@@ -2180,17 +2797,18 @@ void step_kernel(StepArgs a) {
                 const uint32_t type = __builtin_amdgcn_readfirstlane(ph.type);
                 const uint32_t start = __builtin_amdgcn_readfirstlane(ph.start);
                 const uint32_t cnt = __builtin_amdgcn_readfirstlane(ph.count);
+                const bool com = __builtin_amdgcn_readfirstlane(ph.com) != 0u;
                 const JointPhase ph2 = md.jph[p2];
                 {
                     const uint32_t st = __builtin_amdgcn_readfirstlane(ph1.start), cn = __builtin_amdgcn_readfirstlane(ph1.count);
                     nxt = load_half(md.jrec + (st + (kf < cn ? kf : 0u)) * kJRecQuads + half);
                 }
-                if (live && kf < cnt) solve_joint(type, cur, load_jstate(cur, s, odd), md.jrec + (start + kf) * kJRecQuads, s, odd);
+                if (live && kf < cnt) solve_joint(type, com, cur, load_jstate(cur, s), md.jrec + (start + kf) * kJRecQuads, s, odd);
                 if (live) {
                     for (uint32_t k = kf + G / 2; k < cnt; k += G / 2) {
                         const float4* r = md.jrec + (start + k) * kJRecQuads;
                         const JHalf hk = load_half(r + half);
-                        solve_joint(type, hk, load_jstate(hk, s, odd), r, s, odd);
+                        solve_joint(type, com, hk, load_jstate(hk, s), r, s, odd);
                     }
                 }
                 wave_sync<HBM>();
@@ -2215,66 +2833,48 @@ void step_kernel(StepArgs a) {
         }
         const uint32_t my_nlev = live ? s.misc[2] : 0u;
         // ---- I: solve_contacts, iterations x levels (world.zig:1199-1213, S4) --------
-        // Lane pair (2k, 2k+1) takes the k-th slot of each level (and k + G/2, ... when a
-        // level holds more). The level lists and the slots' static parts are read ahead over
-        // the sequence of (iteration, level) steps: at step f the lane's slot record of step
-        // f + 1, its slot index of step f + 2 and the level bounds of step f + 3 are loaded,
-        // so a step starts with its record in registers and reads only the bodies' state.
+        bool spill = false;
+        if constexpr (POOL) spill = __ballot(live && s.misc[1] > a.lds.cap) != 0ull;
         if (do_solve && max_lev > 0) {
-            const bool odd = (sl & 1) != 0;
-            const uint32_t kf = (uint32_t)sl >> 1;
-            const uint32_t nsteps = a.iters * max_lev;
-            // Level bounds of step f: the level's first slot index and its end, read raw (the
-            // lane's slot is first + kf); `ok` when the step exists for the lane's env. The
-            // comparison with the end happens a step later, once the read has landed.
-            auto bounds = [&](uint32_t f, uint32_t lv, uint32_t& first, uint32_t& end) -> bool {
-                first = s.loff[lv - 1];
-                end = s.loff[lv];
-                return f < nsteps && live && lv <= my_nlev;
-            };
-            auto next_lv = [&](uint32_t lv) -> uint32_t { return lv == max_lev ? 1u : lv + 1u; };
-            uint32_t j0, e0, j1, e1, j2, e2;
-            uint32_t lv3 = 1;
-            bool v0 = bounds(0, lv3, j0, e0);
-            lv3 = next_lv(lv3);
-            bool v1 = bounds(1, lv3, j1, e1);
-            lv3 = next_lv(lv3);
-            bool v2 = bounds(2, lv3, j2, e2);
-            lv3 = next_lv(lv3);
-            j0 += kf; v0 = v0 && j0 < e0;
-            j1 += kf; v1 = v1 && j1 < e1;
-            CRec cA = load_crec(s, v0 ? s.lst[j0] : 0u), cB;
-            bool cv = v0;
-            uint32_t ce = e0, cj = j0;
-            uint32_t p1 = v1 ? s.lst[j1] : 0u;
-            // One step with `cur` while the next step's record is loaded into `nxt`; two
-            // steps per trip with the record buffers swapping roles (no record copies).
-            auto cstep = [&](uint32_t f, const CRec& cur, CRec& nxt) {
-                uint32_t j3, e3;
-                const bool ok3 = bounds(f + 3, lv3, j3, e3);
-                lv3 = next_lv(lv3);
-                j2 += kf;
-                v2 = v2 && j2 < e2;
-                const uint32_t p2 = v2 ? s.lst[j2] : 0u;
-                nxt = load_crec(s, p1);
-                if (cv) {
-                    solve_contact_rec(md, s, cur, odd);
-                    for (uint32_t j = cj + G / 2; j < ce; j += G / 2) solve_contact2(md, s, s.lst[j], odd);
+            if constexpr (POOL) {
+                if (!spill) {
+                    solve_contacts<G, true, false>(a, md, s, (float4*)s.con, s.lst, s.loff, live, sl, max_lev, my_nlev);
+                } else {
+                    const SpillArrays sp = spill_arrays(slist, M);
+                    solve_contacts<G, true, true>(a, md, s, (float4*)tlist, sp.lst, sp.loff, live, sl, max_lev, my_nlev);
                 }
-                wave_sync<HBM>();
-                cv = v1; ce = e1; cj = j1;
-                p1 = p2; v1 = v2; e1 = e2; j1 = j2;
-                v2 = ok3; e2 = e3; j2 = j3;
-            };
-            uint32_t f = 0;
-            for (; f + 2 <= nsteps; f += 2) {
-                cstep(f, cA, cB);
-                cstep(f + 1, cB, cA);
+            } else {
+                solve_contacts<G, false, HBM>(a, md, s, nullptr, s.lst, s.loff, live, sl, max_lev, my_nlev);
             }
-            if (f < nsteps) cstep(f, cA, cB);
         }
         tick(PH_CONTACTS);
         if (SPLIT) __syncthreads();  // split barrier 3: the contact list is final for this substep
+        if constexpr (POOL) {
+            // The pool -> the list: the valid slots' records (impulses y and z are 0 in every slot
+            // that is in contact), and "no contact" for the slots that were not marked so yet.
+            if (do_prep && live) {
+                const uint32_t nv = s.misc[1];
+                auto write_valid = [&](const float4* from) {
+                    for (uint32_t i = sl; i < nv; i += G) {
+                        const float4 q0 = from[4 * i], q1 = from[4 * i + 1], q3 = from[4 * i + 3];
+                        ContactRec* const c = &list[fbits(q3.y)];
+                        *(float4*)c->position_pen = q0;
+                        *(float4*)c->normal_friction = q1;
+                        *(float4*)c->impulses = make_float4(q3.z, 0.0f, 0.0f, q3.w);
+                    }
+                };
+                if (spill) write_valid((const float4*)tlist);
+                else write_valid((const float4*)s.con);
+                const uint32_t n_now = count < M ? count : M;
+                for (uint32_t w = 0; w < (M + 63u) / 64u; ++w) {
+                    unsigned long long m = s.wmask[w] & ~s.vmask[w];
+                    if (m == 0ull) continue;
+                    for (uint32_t k = w * 64u + (uint32_t)sl; k < n_now && k < w * 64u + 64u; k += G) {
+                        if (((m >> (k & 63u)) & 1ull) != 0ull) list[k].position_pen[3] = -1.0f;
+                    }
+                }
+            }
+        }
         // ---- J: xpbd_update_velocities (:1922-1961) ----------------------------------
         if (live && do_solve) {
             const float inv_dt = 1.0f / a.dt;
@@ -2429,6 +3029,12 @@ void step_kernel(StepArgs a) {
         }  // do_solve
         if (do_prep) {
         ContactRec* gc = a.contacts + (size_t)env * M;
+        if constexpr (POOL) {
+            if (hv.contacts) {
+                wave_sync<true>();
+                for (uint32_t k = sl; k < n_out; k += G) copy_record(&hv.contacts[(size_t)env * M + k], &list[k]);
+            }
+        } else
         for (uint32_t k = sl; k < n_out; k += G) {
             const float4* src = (const float4*)&s.con[s.perm[k]];
             const float4 c0 = src[0], c1 = src[1], c2 = src[2], c3 = src[3];
@@ -2448,6 +3054,10 @@ void step_kernel(StepArgs a) {
         // Not advanced: keep visible state, record the advanced contact list as the
         // previous-contact snapshot (world.zig:880-928 restores everything else).
         ContactRec* pc = a.prev_out + (size_t)env * M;
+        if constexpr (POOL) {
+            wave_sync<true>();
+            for (uint32_t k = sl; k < n_out; k += G) copy_record(&pc[k], &list[k]);
+        } else
         for (uint32_t k = sl; k < n_out; k += G) {
             const float4* src = (const float4*)&s.con[s.perm[k]];
             float4* d = (float4*)&pc[k];
@@ -2554,6 +3164,8 @@ hipError_t launch_step(const StepArgs& a, int envs_per_wave, int waves, hipStrea
     if ((a.placement >= PL_ALL_HBM) != (a.work != nullptr)) return hipErrorInvalidValue;
     const size_t env_lds = (size_t)a.lds.bytes * (size_t)envs_per_wave;
     const size_t shmem = (size_t)a.ml.bytes + env_lds * (size_t)waves;
+    if (!a.hash && a.placement <= PL_MODEL_HBM && (a.lds.cap == 0 || !a.list_snap || !a.list_tmp || (a.step_mask && !a.list_masked)))
+        return hipErrorInvalidValue;
     // Extended-contact mode with one environment per workgroup: the instance whose narrow
     // phase visits the slots grouped by geom-type pair (same results, less divergence).
     if (a.ext_contacts && a.M >= 64 && envs_per_wave == 1 && !split) {

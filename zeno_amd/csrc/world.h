@@ -40,6 +40,7 @@ struct World {
     bool base_split = false, shape_forced = false;
     int cus = 256;
     EnvLds lds{};
+    EnvLds base_lds{};   // the creation-time shape's working set
     EnvLds lds_small{};  // placement 2: the arrays kept in LDS
     bool hash = false;  // spatial-hash broad phase (more than kHashMinGeoms geoms)
     bool hrows = false;  // hash filter classes fit the model's rows (build_hash_words)
@@ -59,6 +60,9 @@ struct World {
     float *d_jpos = nullptr, *d_jvel = nullptr, *d_jtrq = nullptr, *d_obs = nullptr, *d_lam = nullptr;
     float* d_actions = nullptr;
     ContactRec* d_con = nullptr;
+    // Contact pool (working sets in LDS without the spatial hash): scratch lists of every
+    // environment, and the working lists of environments a step mask holds back (on first use).
+    ContactRec *d_list_snap = nullptr, *d_list_tmp = nullptr, *d_list_masked = nullptr;
     uint32_t *d_counts = nullptr, *d_pcounts = nullptr;
     uint32_t* d_cell_ids = nullptr;       // [E*G] hash mode
     // Count-only sweep of a full list: the non-plane geoms (at most 64; none when the scene
@@ -147,6 +151,7 @@ struct World {
     void set_extended_contacts(bool on);
 
    private:
+    std::vector<uint32_t> pool_sizes() const;
     hipError_t launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask);
     hipError_t stage_actions(const float* actions, const float** d_out);
     hipError_t mark_actions_used();

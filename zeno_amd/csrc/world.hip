@@ -94,7 +94,8 @@ World::~World() {
     release_graph();
     void* dev[] = {d_model, d_phase, d_init_pos, d_init_quat, d_init_vel, d_init_angvel, d_pos, d_quat, d_vel, d_angvel, d_acc,
                    d_jpos, d_jvel, d_jtrq, d_obs, d_lam, d_actions, d_con, d_counts, d_pcounts, d_prev_con,
-                   d_prev_detached, d_mask, d_stage, d_cell_ids, d_work, d_sweep};
+                   d_prev_detached, d_mask, d_stage, d_cell_ids, d_work, d_sweep,
+                   d_list_snap, d_list_tmp, d_list_masked};
     for (void* p : dev) if (p) hipFree(p);
     for (int i = 0; i < MIR_COUNT_ALL; ++i) if (h_mirror[i]) hipHostFree(h_mirror[i]);
     for (int i = 0; i < kStage; ++i) {
@@ -153,6 +154,17 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
 
     w->hash = m.num_geoms > kHashMinGeoms;
     if (w->hash && m.num_geoms > kHashMaxGeoms) { err = "scene too large for the spatial hash (over 16384 geoms)"; delete w; return nullptr; }
+    if (!w->hash && !m.pairs.empty()) {
+        std::vector<uint32_t> sweep;
+        for (uint32_t g = 0; g < m.num_geoms; ++g) if (m.geoms[g].type_body[0] != GEOM_PLANE) sweep.push_back(g);
+        if (!sweep.empty() && sweep.size() <= 64) {
+            for (uint32_t pr : m.pairs) {
+                if (m.geoms[pr & 0xFFFFu].type_body[0] == GEOM_PLANE || m.geoms[pr >> 16].type_body[0] == GEOM_PLANE) ++w->sweep_planes;
+            }
+            w->sweep_n = (uint32_t)sweep.size();
+            if ((e = upload(w, &w->d_sweep, sweep.data(), sweep.size())) != hipSuccess) return fail("upload", e);
+        }
+    }
     EnvLds L = make_env_lds(w->B, w->Jp, w->N, std::max<uint32_t>(w->M, 1), m.num_geoms, 0, false, w->obsp);
     std::vector<float4> invmi(w->B), com(w->B);
     std::vector<uint32_t> flags(w->B);
@@ -201,10 +213,20 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
         L_small = make_env_lds_small(w->B, w->Jp, std::max<uint32_t>(w->M, 1), m.num_geoms, !w->hash, false);
     const EnvLds L_own = make_env_lds(w->B, w->Jp, w->N, std::max<uint32_t>(w->M, 1), m.num_geoms, 16 * kJRecQuads * w->nrec,
                                       !w->hash, w->obsp);
+    // Without the hash, the placements with working sets in LDS keep the contact list in HBM and
+    // a pool of its valid slots in LDS. Each shape is offered with falling pool sizes: a smaller
+    // pool is taken only where it lets more environments be resident (the score below), and none
+    // below kPoolFloor slots or one per body, since a substep with more valid slots than the pool
+    // holds runs its contact solve out of HBM.
+    const std::vector<uint32_t> caps = w->hash ? std::vector<uint32_t>{0u} : w->M > kPoolMaxList ? std::vector<uint32_t>{} : w->pool_sizes();
+    auto pool = [&](uint32_t cap, bool split, bool own) {
+        return make_env_pool(w->B, w->Jp, w->N, std::max<uint32_t>(w->M, 1), cap, split, m.num_geoms,
+                             own ? 16 * kJRecQuads * w->nrec : 0, own, w->sweep_n != 0, w->obsp);
+    };
     // Placement 3: the whole working set in HBM, the hash's staged geoms included.
     const EnvLds L_work = make_env_lds(w->B, w->Jp, w->N, std::max<uint32_t>(w->M, 1), m.num_geoms,
                                        16 * kJRecQuads * w->nrec, !w->hash, w->obsp, true);
-    struct Cand { uint32_t pl; int epw; int waves; size_t shmem; bool split; };
+    struct Cand { uint32_t pl; int epw; int waves; size_t shmem; bool split; EnvLds lds; };
     std::vector<Cand> cands;
     int force_pl = -1, force_epw = 0, force_waves = 0, force_split = -1;
     if (const char* env = std::getenv("ZENO_AMD_PLACEMENT")) force_pl = std::min(std::max(std::atoi(env), 0), 3);
@@ -215,14 +237,19 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     {
         std::vector<int> order;
         for (int cand : {8, 4, 2}) {
-            if (w->hash) continue;
-            if ((size_t)ML.bytes + (size_t)L.bytes * cand > 64 * 1024) continue;
+            if (w->hash || w->B > 2u * (64u / (uint32_t)cand)) continue;
+            if (caps.empty() || (size_t)ML.bytes + (size_t)pool(caps.back(), true, false).bytes * cand > 64 * 1024) continue;
             if ((w->E + cand - 1) / cand < 1024) continue;
             order.push_back(cand);
             break;
         }
         for (int cand : {1, 2, 4, 8}) {
             if (cand > 1 && w->hash) continue;
+            // At most two bodies per lane, unless the shape is forced: the stages over bodies and
+            // slots take a pass per lane's share of them (the 65-body pile at eight environments
+            // per wave and one wave on each SIMD takes 4.0 ms where one environment per wave and
+            // eight waves, as many environments, take 0.6 ms).
+            if (cand > 1 && force_epw != cand && w->B > 2u * (64u / (uint32_t)cand)) continue;
             if (std::find(order.begin(), order.end(), cand) == order.end()) order.push_back(cand);
         }
         for (bool split : {true, false}) {
@@ -230,17 +257,23 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
             for (int waves : {4, 1, 2}) {
                 if (waves > 1 && w->hash) continue;
                 for (int cand : order) {
-                    const size_t shmem = (size_t)ML.bytes + (size_t)L.bytes * cand * waves;
-                    if (shmem <= lds_max) cands.push_back({PL_LDS, cand, waves, shmem, split});
+                    for (uint32_t cap : caps) {
+                        const EnvLds l = w->hash ? L : pool(cap, split, false);
+                        const size_t shmem = (size_t)ML.bytes + (size_t)l.bytes * cand * waves;
+                        if (shmem <= lds_max) cands.push_back({PL_LDS, cand, waves, shmem, split, l});
+                    }
                 }
             }
         }
-        if ((size_t)L_own.bytes <= lds_max) cands.push_back({PL_MODEL_HBM, 1, 1, (size_t)L_own.bytes, false});
-        cands.push_back({PL_ALL_HBM, 1, 1, (size_t)L_small.bytes, false});
+        for (uint32_t cap : caps) {
+            const EnvLds l = w->hash ? L_own : pool(cap, false, true);
+            if ((size_t)l.bytes <= lds_max) cands.push_back({PL_MODEL_HBM, 1, 1, (size_t)l.bytes, false, l});
+        }
+        cands.push_back({PL_ALL_HBM, 1, 1, (size_t)L_small.bytes, false, L_own});
     }
     // Placement 3 (no LDS at all) is the fallback for contact lists that no LDS layout
     // holds: it scores well on residency, but its contact pipeline runs out of the caches.
-    const std::vector<Cand> fallback{{PL_WORK_HBM, 1, 1, 0, false}};
+    const std::vector<Cand> fallback{{PL_WORK_HBM, 1, 1, 0, false, L_work}};
     const Cand* best = nullptr;
     uint64_t best_score = 0;
     for (int pass = 0; pass < 2 && !best; ++pass) {
@@ -264,9 +297,8 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     }
     w->placement = best->pl;
     const int epw = best->epw;
-    if (best->pl == PL_MODEL_HBM || best->pl == PL_ALL_HBM) L = L_own;
-    if (best->pl == PL_WORK_HBM) L = L_work;
-    w->lds = L;
+    w->lds = best->lds;
+    w->base_lds = best->lds;
     w->lds_small = L_small;
     w->epw = epw;
     w->waves = best->waves;
@@ -307,17 +339,6 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
         }
         if ((e = upload(w, &w->d_model, (const uint4*)blob.data(), w->ml.bytes / 16)) != hipSuccess) return fail("upload", e);
     }
-    if (!w->hash && !m.pairs.empty()) {
-        std::vector<uint32_t> sweep;
-        for (uint32_t g = 0; g < m.num_geoms; ++g) if (m.geoms[g].type_body[0] != GEOM_PLANE) sweep.push_back(g);
-        if (!sweep.empty() && sweep.size() <= 64) {
-            for (uint32_t pr : m.pairs) {
-                if (m.geoms[pr & 0xFFFFu].type_body[0] == GEOM_PLANE || m.geoms[pr >> 16].type_body[0] == GEOM_PLANE) ++w->sweep_planes;
-            }
-            w->sweep_n = (uint32_t)sweep.size();
-            if ((e = upload(w, &w->d_sweep, sweep.data(), sweep.size())) != hipSuccess) return fail("upload", e);
-        }
-    }
     std::vector<float4> ip(w->B), iq(w->B), iv(w->B), ia(w->B);
     for (uint32_t b = 0; b < w->B; ++b) {
         ip[b] = make_float4(m.init_pos[4 * b], m.init_pos[4 * b + 1], m.init_pos[4 * b + 2], m.init_pos[4 * b + 3]);
@@ -349,6 +370,10 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     if ((e = dalloc(w, &w->d_counts, w->E)) != hipSuccess) return fail("hipMalloc", e);
     if ((e = dalloc(w, &w->d_pcounts, w->E)) != hipSuccess) return fail("hipMalloc", e);
     if (w->hash && (e = dalloc(w, &w->d_cell_ids, (size_t)w->E * m.num_geoms)) != hipSuccess) return fail("hipMalloc", e);
+    if (!w->hash && w->placement <= PL_MODEL_HBM) {
+        if ((e = dalloc(w, &w->d_list_snap, (size_t)w->E * std::max<uint32_t>(w->M, 1))) != hipSuccess) return fail("hipMalloc", e);
+        if ((e = dalloc(w, &w->d_list_tmp, (size_t)w->E * std::max<uint32_t>(w->M, 1))) != hipSuccess) return fail("hipMalloc", e);
+    }
     if (w->placement >= PL_ALL_HBM && (e = dalloc(w, &w->d_work, (size_t)w->E * w->lds.bytes)) != hipSuccess) return fail("hipMalloc", e);
     struct Z { void* p; size_t n; } zeros[] = {
         {w->d_pos, EB * 16}, {w->d_quat, EB * 16}, {w->d_vel, EB * 16}, {w->d_angvel, EB * 16}, {w->d_acc, EB * 16},
@@ -433,6 +458,9 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
     a.contacts = d_con; a.counts = d_counts; a.pcounts = d_pcounts;
     a.prev_detached = d_prev_detached;
     a.prev_contacts = d_prev_con;
+    a.list_snap = d_list_snap;
+    a.list_tmp = d_list_tmp;
+    a.list_masked = d_list_masked;
     a.step_mask = d_step_mask;
     a.prev_out = d_prev_con;
     a.prev_detached_out = d_prev_detached;
@@ -524,6 +552,22 @@ hipError_t World::step(const float* actions, uint32_t substeps, bool actions_on_
     return refresh_views();
 }
 
+// Pool sizes offered to the launch shapes, largest first: the whole list, then fewer slots.
+// ZENO_AMD_POOL=n (tests of pools that overflow) offers n alone.
+std::vector<uint32_t> World::pool_sizes() const {
+    if (const char* env = std::getenv("ZENO_AMD_POOL")) {
+        const int n = std::atoi(env);
+        if (n > 0) return {std::min((uint32_t)n, std::max<uint32_t>(M, 1))};
+    }
+    const uint32_t m = std::max<uint32_t>(M, 1), floor = std::min(m, std::max(kPoolFloor, (B + 7u) & ~7u));
+    std::vector<uint32_t> sizes{m};
+    for (uint32_t c : {512u, 256u, 192u, 128u, 96u, 64u, 48u, 32u, 24u}) {
+        if (c < m && c >= floor) sizes.push_back(c);
+    }
+    if (sizes.back() > floor) sizes.push_back(floor);
+    return sizes;
+}
+
 void World::set_extended_contacts(bool on) {
     release_graph();
     ext_contacts = on;
@@ -531,20 +575,26 @@ void World::set_extended_contacts(bool on) {
     epw = base_epw;
     waves = base_waves;
     split = base_split;
+    lds = base_lds;
     if (!on || M < 64) return;
     // The grouped narrow phase runs in the one-environment-per-wave instances without split
     // groups: the best of those by resident environments (the creation-time score).
     uint64_t best = 0;
     for (int w : {4, 1, 2}) {
-        const size_t shmem = (size_t)ml.bytes + (size_t)lds.bytes * (size_t)w;
-        const int n = resident_workgroups(1, PL_LDS, false, shmem, w, false);
-        if (n <= 0) continue;
-        const uint64_t score = std::min<uint64_t>(E, (uint64_t)n * (uint64_t)w * (uint64_t)cus);
-        if (score > best) {
-            best = score;
-            epw = 1;
-            waves = w;
-            split = false;
+        for (uint32_t cap : pool_sizes()) {
+            const EnvLds l = make_env_pool(B, Jp, N, M, cap, false, model.num_geoms, 0, false, false, obsp);
+            const size_t shmem = (size_t)ml.bytes + (size_t)l.bytes * (size_t)w;
+            if (shmem > max_lds_per_workgroup(device)) continue;
+            const int n = resident_workgroups(1, PL_LDS, false, shmem, w, false);
+            if (n <= 0) continue;
+            const uint64_t score = std::min<uint64_t>(E, (uint64_t)n * (uint64_t)w * (uint64_t)cus);
+            if (score > best) {
+                best = score;
+                epw = 1;
+                waves = w;
+                split = false;
+                lds = l;
+            }
         }
     }
 }
@@ -603,6 +653,7 @@ hipError_t World::graph_launch() {
 }
 
 hipError_t World::ensure_subset_buffers() {
+    if (d_list_snap && !d_list_masked) ZA_TRY(dalloc(this, &d_list_masked, (size_t)E * std::max<uint32_t>(M, 1)));
     if (!d_prev_con) {
         release_graph();  // captured launches hold the buffer addresses of capture time
         ZA_TRY(dalloc(this, &d_prev_con, (size_t)E * std::max<uint32_t>(M, 1)));
