@@ -86,6 +86,44 @@ def test_multi_substep_replay_matches_oracle():
         buf.free()
 
 
+@pytest.mark.parametrize("name,envs,steps,substeps", [("pendulum", 5, 1, 1), ("humanoid", 19, 65, 1), ("hash_terrain", 3, 5, 2),
+                                                      ("pile_hash", 2, 4, 1), ("walker", 9, 130, 3)])
+def test_fused_steps_match_the_oracle(name, envs, steps, substeps):
+    """Captured launches run up to 64 steps each: schedules around that length, more actions than
+    lanes, and working sets in HBM, replayed twice with an eager step between."""
+    g, o, acts = make_pair(name, envs, 2 * steps + 1, seed=17) if name != "walker" else walker_pair(envs, 2 * steps + 1)
+    A = g.action_dim
+    buf = DeviceBuffer(np.ascontiguousarray(acts, np.float32).reshape(-1))
+    try:
+        g.capture_steps(buf.ptr.value, envs * A * 4, steps, substeps)
+        for replay in range(2):
+            g.graph_launch()
+            for k in range(steps):
+                o.step(acts[k], substeps=substeps)
+            compare(gpu_arrays(g), oracle_arrays(o), 0.0, 0.0)
+            g.step(acts[2 * steps], 1)
+            o.step(acts[2 * steps], substeps=1)
+        compare(gpu_arrays(g), oracle_arrays(o), 0.0, 0.0)
+    finally:
+        g.release_graph()
+        buf.free()
+
+
+def walker_pair(envs, steps):
+    from oracle.oracle import OracleWorld
+    from zeno_amd.model import load_model
+    from zeno_amd.scenes import ASSETS, actions, initial_state
+    from zeno_amd.world import ZenoWorld
+
+    path = str(ASSETS / "walker.xml")
+    model = load_model(mjcf_path=path)
+    state = initial_state(model, envs, 0.1, 0.0, 0.1, 18)
+    g, o = ZenoWorld(mjcf_path=path, num_envs=envs), OracleWorld(model, envs)
+    for w in (g, o):
+        w.reset_to_state(*state)
+    return g, o, actions(envs, model["num_actuators"], steps, 1.0, 19)
+
+
 def test_setters_release_the_graph():
     g, _, acts = make_pair("pendulum", 8, 2, seed=13)
     buf = DeviceBuffer(np.ascontiguousarray(acts, np.float32).reshape(-1))

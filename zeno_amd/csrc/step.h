@@ -459,6 +459,10 @@ struct StepArgs {
     const uint32_t* sweep;
     uint32_t sweep_n, sweep_planes;
     uint32_t iters, substeps;
+    // Consecutive steps in this launch, step k reading its actions action_stride bytes after
+    // step k - 1's (a captured schedule; 1 otherwise).
+    uint32_t calls;
+    uint64_t action_stride;
     // Scalars (SimParams, world.zig:35-56).
     float dt, inv_step, gx, gy, gz, restitution, baumgarte, slop;
     // Model blob (read-only, one copy per world), laid out by `ml`.

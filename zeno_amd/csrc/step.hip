@@ -1517,7 +1517,10 @@ void step_kernel(StepArgs a) {
     uint32_t count = 0, pcount = 0;
     bool detached = false;
     // The lane's first action (read by stage A of every substep) is loaded with the state.
-    const float act0 = (live && do_solve && (uint32_t)sl < a.A) ? a.actions[(size_t)env * a.A + sl] : 0.0f;
+    // With several calls in the launch the next call's are read while this one runs.
+    const float* acts = a.actions;
+    auto first_action = [&](const float* from) { return (live && do_solve && (uint32_t)sl < a.A) ? from[(size_t)env * a.A + sl] : 0.0f; };
+    float act0 = first_action(acts), act_next = 0.0f;
     const size_t eb = (size_t)env * B;
     const ContactRec* gc = a.contacts + (size_t)env * M;
     const uint32_t b0 = sl, j0 = sl;
@@ -1700,7 +1703,18 @@ void step_kernel(StepArgs a) {
 
     const int lane_of_env = sl;
     const Lds launch_s = s;
-    for (uint32_t step = 0; step < a.substeps; ++step) {
+    // A launch runs `calls` consecutive steps (zeno_world_step calls) of `substeps` each. Between
+    // two of them nothing leaves the working sets: the state, the observations and the
+    // accelerations a caller can see are those after the last.
+    const uint32_t total = a.calls * a.substeps;
+    uint32_t in_call = 0;  // substep within its call
+    for (uint32_t step = 0; step < total; ++step) {
+        if (in_call == a.substeps) {
+            in_call = 0;
+            acts = (const float*)((const char*)acts + a.action_stride);
+            act0 = act_next;
+        }
+        if (in_call == 0 && step + a.substeps < total) act_next = first_action((const float*)((const char*)acts + a.action_stride));
         // Opaque in each substep, so that the addresses that follow from the lane are formed where
         // they are used: hoisted out of this loop they are some fifty registers, which the compiler
         // spills to scratch.
@@ -1772,7 +1786,7 @@ void step_kernel(StepArgs a) {
         const bool snap_first = LATE_SNAP && (uint64_t)count + (uint64_t)a.G * (uint64_t)(a.G - 1u) / 2u > 0xFFFFFFFFull;
         if (!POOL && (!LATE_SNAP || snap_first) && live) snapshot(M, snap_first ? hppen : s.ppen, snap_first ? hpimp : s.pimp);
         // Stage B (below), one text for the two places it runs from.
-        const bool take_vb = alias && step == 0;  // aliased: the velocity at call start
+        const bool take_vb = (alias || step > 0) && in_call == 0;  // the velocity at call start, where the load did not set it
         auto stage_b = [&]() {
             if (bf != 0u && sl == 0) {
                 s.frc[0] = make_float4(0, 0, 0, 0);
@@ -1818,7 +1832,7 @@ void step_kernel(StepArgs a) {
             for (uint32_t i = sl; i < N; i += G) s.lam[i] = 0.8f * s.lam[i];
             for (uint32_t k = sl; k < a.A; k += G) {
                 const ActuatorRec& act = md.acts[k];
-                const float av = k == (uint32_t)sl ? act0 : a.actions[(size_t)env * a.A + k];
+                const float av = k == (uint32_t)sl ? act0 : acts[(size_t)env * a.A + k];
                 float ctrl = clampf(av, act.params[1], act.params[2]);
                 float torque = clampf(ctrl * act.params[3], act.params2[0], act.params2[1]);
                 s.jt[(uint32_t)act.params[0]] = torque;
@@ -1928,7 +1942,7 @@ void step_kernel(StepArgs a) {
                 q4 dq = qmul(toq(tof4(q)), qconj(toq(Q)));
                 if (dq.w < 0) dq = qneg(dq);
                 s.angvel[b] = tof4(scale(sscale(2.0f, xyz(dq)), inv_dt), 0.0f);
-                if (j_acc && step + 1 == a.substeps) {
+                if (j_acc && step + 1 == total) {
                     const float4 v0 = take_vb ? V : s.vb[b];
                     a.acc[(size_t)env * B + b] = make_float4((v.x - v0.x) * a.inv_step, (v.y - v0.y) * a.inv_step, (v.z - v0.z) * a.inv_step, 0.0f);
                 }
@@ -2878,7 +2892,7 @@ void step_kernel(StepArgs a) {
         // ---- J: xpbd_update_velocities (:1922-1961) ----------------------------------
         if (live && do_solve) {
             const float inv_dt = 1.0f / a.dt;
-            const bool acc_here = j_acc && step + 1 == a.substeps;
+            const bool acc_here = j_acc && step + 1 == total;
             uint32_t kb = 0;
             for (uint32_t b = bf + sl; b < B; b += G, ++kb) {
                 if (HBM && ((early_bits >> kb) & 1u) != 0u) continue;
@@ -2936,7 +2950,7 @@ void step_kernel(StepArgs a) {
         // ---- L: read_sensors (:1799-1893); cache_contacts is the next snapshot --------
         // The row is assembled in the working set and written back with the state. Entries
         // that no sensor writes are 0 (nothing else ever writes the observation buffer).
-        if (stepped && do_solve && step + 1 == a.substeps) {
+        if (stepped && do_solve && step + 1 == total) {
             float* obs = s.obs;
             for (uint32_t k = sl; k < a.obsp; k += G) obs[k] = 0.0f;
             wave_sync<HBM>();
@@ -2961,6 +2975,7 @@ void step_kernel(StepArgs a) {
             }
         }
         pcount = count;
+        ++in_call;
         wave_sync<HBM>();
         tick(PH_POST);
     }

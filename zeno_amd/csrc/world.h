@@ -120,6 +120,7 @@ struct World {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     uint32_t graph_steps = 0;
+    static constexpr uint32_t kFusedCalls = 64;  // steps per captured launch
     bool capturing = false;
 
     ~World();
@@ -152,7 +153,7 @@ struct World {
 
    private:
     std::vector<uint32_t> pool_sizes() const;
-    hipError_t launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask);
+    hipError_t launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask, uint32_t calls = 1, uint64_t action_stride = 0);
     hipError_t stage_actions(const float* actions, const float** d_out);
     hipError_t mark_actions_used();
     hipError_t upload_mask(const uint8_t* mask, uint8_t** d_out);

@@ -428,7 +428,7 @@ hipError_t World::sync() { return hipStreamSynchronize(stream); }
 
 uint64_t World::state_bytes() const { return device_bytes; }
 
-hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask) {
+hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask, uint32_t calls, uint64_t action_stride) {
     StepArgs a{};
     a.E = E; a.B = B; a.J = J; a.Jp = Jp; a.A = A; a.S = model.num_sensors; a.obsp = obsp; a.N = N;
     a.nrec = nrec; a.njph = njph; a.M = M; a.P = model.num_pairs;
@@ -444,6 +444,7 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
     a.placement = placement;
     a.work = d_work;
     a.iters = iters; a.substeps = substeps;
+    a.calls = calls; a.action_stride = action_stride;
     a.dt = dt;
     a.inv_step = timestep > 0 ? 1.0f / timestep : 0.0f;
     a.gx = gravity[0]; a.gy = gravity[1]; a.gz = gravity[2];
@@ -611,8 +612,12 @@ void World::release_graph() {
 
 // `steps` consecutive steps, step k reading its actions at d_actions + k * stride_bytes,
 // captured from the world's stream into one HIP graph: a replay is one launch call for the
-// whole sequence instead of one per step. Every node is a step-kernel launch (no memset or
-// copy nodes). Substeps, dt, gravity, the contact mode and the buffer addresses are fixed at
+// whole sequence. Environments do not meet within a step, so a launch takes kFusedCalls steps
+// one after another without storing and reloading the state between them, and an environment
+// with many contacts in one step holds no other up: a node per kFusedCalls steps instead of per
+// step (Ant, 4096 environments, 32 steps: 2041 -> 1370 us; the bound keeps a launch of the
+// slowest scenes well under a second). Every node is a step-kernel launch (no memset or copy
+// nodes). Substeps, dt, gravity, the contact mode and the buffer addresses are fixed at
 // capture; the world's setters for them release the graph.
 hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint32_t steps, uint32_t substeps) {
     ZA_TRY(hipSetDevice(device));
@@ -623,10 +628,10 @@ hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint3
     ZA_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     capturing = true;
     hipError_t e = hipSuccess;
-    for (uint32_t k = 0; k < steps && e == hipSuccess; ++k) {
+    for (uint32_t k = 0; k < steps && e == hipSuccess; k += kFusedCalls) {
         const float* a = A > 0 ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(d_act) + k * stride_bytes)
                                : d_actions;
-        e = launch(a, actual, nullptr);
+        e = launch(a, actual, nullptr, std::min(kFusedCalls, steps - k), A > 0 ? stride_bytes : 0);
     }
     capturing = false;
     hipGraph_t g = nullptr;
