@@ -455,7 +455,9 @@ struct StepArgs {
     // host changed the counts, exposing slots whose order the last sort did not cover).
     uint32_t sort_all;
     // Count-only broad phase of a full list (one environment per wave): the non-plane geoms
-    // (sweep_n <= 64, else 0 and the sweep is off) and the number of listed pairs with a plane.
+    // (sweep_n <= 64, else 0 and the sweep is off), from entry 64 on a filter word for each (bit
+    // k - 1: the pair with the geom k lanes along is listed, each pair with one of its two lanes),
+    // and the number of listed pairs with a plane.
     const uint32_t* sweep;
     uint32_t sweep_n, sweep_planes;
     uint32_t iters, substeps;

@@ -2136,32 +2136,32 @@ void step_kernel(StepArgs a) {
             // one-lane rotations of the wave each lane holds the geom k lanes along, so
             // k = 1..32 meets every unordered pair once (k = 32 from the lower half only). Each
             // pair takes the list's filters (different bodies, contype / conaffinity; the list
-            // holds exactly the pairs passing them, model.cpp) and the same distance test: the
-            // difference's sign does not change its square, nor the radii's order their sum.
-            const bool mine = (uint32_t)sl < a.sweep_n;
+            // holds exactly the pairs passing them, model.cpp), which do not change: bit k - 1 of
+            // the lane's filter word, from the host, is pair k's. Each pair then takes the same
+            // distance test: the difference's sign does not change its square, nor the radii's
+            // order their sum. Four rotated registers and about 14 other instructions a pair, where
+            // rotating and testing bodies and masks took 7 and 24.
             f3 c = mk3(0.0f, 0.0f, 0.0f);
             float r = 0.0f;
-            uint32_t body = 0, grp = 0, msk = 0;  // an empty lane passes no mask test
-            if (mine) {
+            uint32_t listed = 0;  // an empty lane has no pairs
+            if ((uint32_t)sl < a.sweep_n) {
                 const GeomRec& gr = md.geoms[a.sweep[sl]];
                 c = add(xyz(s.pos[gr.type_body[1]]), mk3(gr.pos_size0[0], gr.pos_size0[1], gr.pos_size0[2]));
                 r = gr.pos_size0[3];
-                body = gr.type_body[1]; grp = gr.type_body[3]; msk = gr.type_body[2];
+                listed = a.sweep[64 + sl];
             }
-            auto rol = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x134, 0xF, 0xF, false); };  // wave_rol:1
-            auto rolf = [&](float v) { return __int_as_float((int)rol((uint32_t)__float_as_int(v))); };
+            auto rolf = [&](float v) {  // wave_rol:1
+                return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x134, 0xF, 0xF, false));
+            };
             float px = c.x, py = c.y, pz = c.z, pr = r;
-            uint32_t pb = body, pg = grp, pm = msk, hits = 0;
-#pragma unroll 4
-            for (uint32_t k = 1; k <= 32u; ++k) {
+            uint32_t hits = 0;
+#pragma unroll 8
+            for (uint32_t k = 0; k < 32u; ++k) {
                 px = rolf(px); py = rolf(py); pz = rolf(pz); pr = rolf(pr);
-                pb = rol(pb); pg = rol(pg); pm = rol(pm);
                 const f3 diff = sub(mk3(px, py, pz), c);
                 const float min_dist = r + pr + 0.1f;
                 const bool near = !(dot(diff, diff) >= min_dist * min_dist);  // NaN distances pass, as in :521
-                const bool listed = body != pb && ((grp & pm) != 0u || (pg & msk) != 0u);
-                const bool once = k < 32u || (uint32_t)sl < 32u;
-                hits += (near && listed && once) ? 1u : 0u;
+                hits += near ? (listed >> k) & 1u : 0u;
             }
             for (uint32_t d = 1; d < 64u; d <<= 1) hits += (uint32_t)__shfl_xor((int)hits, (int)d);
             count += a.sweep_planes + hits;

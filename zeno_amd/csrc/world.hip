@@ -162,6 +162,17 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
                 if (m.geoms[pr & 0xFFFFu].type_body[0] == GEOM_PLANE || m.geoms[pr >> 16].type_body[0] == GEOM_PLANE) ++w->sweep_planes;
             }
             w->sweep_n = (uint32_t)sweep.size();
+            std::vector<uint32_t> lane(m.num_geoms, 64u);
+            for (size_t i = 0; i < sweep.size(); ++i) lane[sweep[i]] = (uint32_t)i;
+            sweep.resize(128, 0u);  // then a filter word per lane
+            for (uint32_t pr : m.pairs) {
+                const uint32_t x = lane[pr & 0xFFFFu], y = lane[pr >> 16];
+                if (x == 64u || y == 64u) continue;  // with a plane
+                // From the lane that meets the other after at most 32 rotations, the lower half's at 32.
+                const uint32_t ahead = (y - x) & 63u;  // lanes from x along to y
+                const bool from_x = ahead < 32u || (ahead == 32u && x < 32u);
+                sweep[64 + (from_x ? x : y)] |= 1u << ((from_x ? ahead : 64u - ahead) - 1u);
+            }
             if ((e = upload(w, &w->d_sweep, sweep.data(), sweep.size())) != hipSuccess) return fail("upload", e);
         }
     }
