@@ -25,13 +25,16 @@ namespace {
 
 // reset (world.zig:1296-1310 with state.zig:390-411): restore the captured initial body
 // state and zero joint positions / velocities of the selected envs.
+// With `counts`, also zeroes every env's contact count, whatever the mask.
 __global__ void reset_envs_kernel(uint32_t E, uint32_t B, uint32_t J, uint32_t Jp, const uint8_t* mask,
                                   const float4* ipos, const float4* iquat, const float4* ivel, const float4* iang,
-                                  float4* pos, float4* quat, float4* vel, float4* ang, float* jpos, float* jvel) {
+                                  float4* pos, float4* quat, float4* vel, float4* ang, float* jpos, float* jvel,
+                                  uint32_t* counts) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;  // E (B + J) may pass 2^32
     const uint32_t per = B + J;
     if (i >= (uint64_t)E * per) return;
     const uint32_t e = (uint32_t)(i / per), k = (uint32_t)(i % per);
+    if (k == 0u && counts) counts[e] = 0u;
     if (mask && !mask[e]) return;
     if (k < B) {
         const size_t o = (size_t)e * B + k;
@@ -397,7 +400,7 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     // initializeState (world.zig:663-691): every env starts from the scene pose.
     hipLaunchKernelGGL(reset_envs_kernel, dim3(blocks_for((uint64_t)w->E * (w->B + w->J), 256)), dim3(256), 0, w->stream,
                        w->E, w->B, w->J, w->Jp, (const uint8_t*)nullptr, w->d_init_pos, w->d_init_quat, w->d_init_vel,
-                       w->d_init_angvel, w->d_pos, w->d_quat, w->d_vel, w->d_angvel, w->d_jpos, w->d_jvel);
+                       w->d_init_angvel, w->d_pos, w->d_quat, w->d_vel, w->d_angvel, w->d_jpos, w->d_jvel, (uint32_t*)nullptr);
     if ((e = hipGetLastError()) != hipSuccess) return fail("init kernel", e);
 
     // Host mirrors: pinned, mapped and coherent, so that the step kernel can store the
@@ -719,10 +722,12 @@ hipError_t World::reset(const uint8_t* mask) {
     ZA_TRY(upload_mask(mask, &dm));
     hipLaunchKernelGGL(reset_envs_kernel, dim3(blocks_for((uint64_t)E * (B + J), 256)), dim3(256), 0, stream,
                        E, B, J, Jp, (const uint8_t*)dm, d_init_pos, d_init_quat, d_init_vel, d_init_angvel,
-                       d_pos, d_quat, d_vel, d_angvel, d_jpos, d_jvel);
+                       d_pos, d_quat, d_vel, d_angvel, d_jpos, d_jvel, d_counts);
     ZA_TRY(hipGetLastError());
-    ZA_TRY(fill_u32(stream, d_counts, E, 0));
-    mark_all_dirty();
+    // Only these mirrors fall behind: a loop that holds the observations alone, and resets some
+    // environments before each step, copies and waits for nothing here (3001 walkers, 1.6% reset
+    // before each step: 111 -> 73 us a pass).
+    for (MirrorId id : {MIR_POS, MIR_QUAT, MIR_VEL, MIR_ANGVEL, MIR_JPOS, MIR_JVEL, MIR_COUNT}) dirty[id] = true;
     return refresh_views();
 }
 
