@@ -146,6 +146,64 @@ def test_hash_filter_classes(classes, placement):
     g.close()
 
 
+@pytest.mark.parametrize("placement", [None, 2, 3])
+@pytest.mark.parametrize("layout", ["flat", "stacked", "crowd", "far_edge", "wild"])
+def test_hash_count_only_layouts(layout, placement):
+    """The count-only queries of a full list (four slots, full after the first step) where their
+    walk takes another form: bodies in one layer of cells (the two runs of a geom's own layer),
+    seven layers (all five runs), three quarters of them in the clamped corner cell and the rest
+    far apart (candidates dealt out across the wave), the clamped far edge (x and y in cell 63,
+    empty runs), and NaN and infinite positions, whose pairs pass or fail the distance test as
+    the reference's comparison has it. Counts, cell ids and state against the oracle."""
+    import os
+    from oracle.oracle import OracleWorld
+    from zeno_amd.model import load_model
+    from zeno_amd.scenes import pile_initial_state, pile_mjcf
+    from zeno_amd.world import ZenoWorld
+    bodies, E = 530, 2
+    xml = pile_mjcf(bodies, seed=5, xy=(-3.0, 12.0))
+    m = load_model(mjcf_string=xml)
+    saved = os.environ.get("ZENO_AMD_PLACEMENT")
+    if placement is not None:
+        os.environ["ZENO_AMD_PLACEMENT"] = str(placement)
+    try:
+        g = ZenoWorld(mjcf_string=xml, num_envs=E, max_contacts_per_env=4)
+    finally:
+        os.environ.pop("ZENO_AMD_PLACEMENT", None)
+        if saved is not None:
+            os.environ["ZENO_AMD_PLACEMENT"] = saved
+    assert g.modes()["spatial_hash"]
+    o = OracleWorld(m, E, max_contacts_per_env=4)
+    pos, *rest = pile_initial_state(m, E, 11, xy=(-3.0, 12.0))
+    rng = np.random.default_rng(17)
+    p = pos[:, 1:, :3]
+    n = p.shape[1]
+    if layout == "flat":
+        p[..., 2] = rng.uniform(0.3, 0.7, p.shape[:2])
+    elif layout == "stacked":
+        p[:] = rng.uniform([0.0, 0.0, 0.2], [8.0, 8.0, 7.0], p.shape)
+    elif layout == "crowd":
+        p[:] = rng.uniform(2.0, 60.0, p.shape)
+        p[:, : 3 * n // 4] = rng.uniform(-8.0, 0.9, (E, 3 * n // 4, 3))
+    elif layout == "far_edge":
+        p[:] = rng.uniform([58.0, 58.0, 59.0], [72.0, 72.0, 70.0], p.shape)
+    else:
+        p[:, ::40] = np.nan
+        p[:, 1::50, 0] = np.inf
+        p[:, 2::50, 1] = -np.inf
+    state = (pos, *rest)
+    g.reset_to_state(*state)
+    o.reset_to_state(*state)
+    G = m["num_geoms"]
+    for k in range(4):
+        g.step(np.zeros((E, 0), np.float32))
+        o.step(None)
+        compare(gpu_arrays(g), oracle_arrays(o), rtol=1e-4, atol=1e-4)
+        np.testing.assert_array_equal(g.get_cell_ids(), o.cell_ids[:, :G], err_msg=f"cell ids, step {k}")
+        assert (o.contact_counts >= 4).all()  # full: the next step only counts
+    g.close()
+
+
 @pytest.mark.parametrize("placement", [None, 2])
 def test_hash_snapshot_after_count_changes(placement):
     """The previous-contact snapshot when the counts drop between calls: after a reset (every

@@ -21,6 +21,8 @@
 // list is written back.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dmath.h"
 #include "narrow_ext.h"
 #include "step.h"
@@ -881,6 +883,36 @@ __device__ __forceinline__ bool hash_filter_pass(const StepArgs& a, const Mdl& m
     return ((fa.x & gr.type_body[2]) | (gr.type_body[3] & fa.y)) != 0u;
 }
 
+// Centre and reach of a geom: its radius, or NaN for a plane, with which the distance test below
+// passes for every other geom, as a pair with a plane does (the staged copy holds it so).
+template <bool STAGED, int BS>
+__device__ __forceinline__ float4 hash_geom_reach(const Mdl& md, const LdsT<BS>& s, const uint32_t* hmeta, uint32_t g) {
+    float4 p = hash_geom_pos<STAGED>(md, s, g);
+    if (!STAGED && hw_plane(hash_geom_meta<STAGED>(md, hmeta, g))) p.w = __builtin_nanf("");
+    return p;
+}
+// Wave scans on DPP (all 64 lanes active): shifts within rows of 16, then the last lane of a row
+// onto the next (row_bcast:15, rows 1 and 3) and of the lower half onto the upper (row_bcast:31).
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    auto up = [&](int t) { v = (uint32_t)t > v ? (uint32_t)t : v; };
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    up(__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+
 template <bool STAGED, int BS>
 __device__ __forceinline__ uint32_t hash_pairs_of(const StepArgs& a, const Mdl& md, const LdsT<BS>& s, const uint32_t* hmeta, uint32_t g, bool emit,
                                   uint32_t slot) {
@@ -967,7 +999,7 @@ __device__ __forceinline__ uint32_t hash_pairs_of(const StepArgs& a, const Mdl& 
 // tests are those of hash_pairs_of; each is symmetric in its two geoms (the difference's
 // sign does not change its square, nor the radii's order their sum), so the earlier geom
 // may take either role. The runs' nine ends are found by interleaved binary searches; then
-// each lane walks its own candidates, or, when one lane holds more than twice the mean, the
+// each lane walks its own candidates, or, when one lane holds far more than the mean, the
 // wave's candidates are dealt out four per lane at a time, each lane finding its candidate's
 // run by a search over the lanes' prefix sums, so a crowded cell does not hold the wave up.
 template <bool STAGED, int BS>
@@ -1027,70 +1059,54 @@ __device__ __forceinline__ uint32_t hash_count_forward(const StepArgs& a, const 
 #pragma unroll
         for (int k = 0; k < R; ++k) n += rl[k];
         // Inclusive prefix over the wave's lanes; T candidates this round.
-        uint32_t inc = n;
-        for (int d = 1; d < kWave; d <<= 1) {
-            const uint32_t t = (uint32_t)__shfl_up((int)inc, d);
-            if (lane >= d) inc += t;
-        }
-        const uint32_t T = (uint32_t)__shfl((int)inc, kWave - 1);
-        const float4 pa4 = mine ? hash_geom_pos<STAGED>(md, s, ga) : make_float4(0, 0, 0, 0);
+        const uint32_t inc = wave_scan_add(n);
+        const uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
+        const float4 pa4 = mine ? hash_geom_reach<STAGED>(md, s, hmeta, ga) : make_float4(0, 0, 0, 0);
         const uint32_t wa = mine ? hash_geom_meta<STAGED>(md, hmeta, ga) : 0u;
         const uint2 fa = mine ? hash_filter_of(a, md, ga, wa) : make_uint2(0u, 0u);
-        // Balanced rounds (no lane with more than twice the mean's chunks) walk each lane's own
-        // runs; others deal the candidates out.
-        uint32_t nmax = n;
-        for (int d = 1; d < kWave; d <<= 1) {
-            const uint32_t t = (uint32_t)__shfl_xor((int)nmax, d);
-            nmax = t > nmax ? t : nmax;
-        }
-        if (nmax <= 2u * ((T + kWave - 1u) / kWave)) {
+        // Rounds where no lane has more than kDealOver times the mean walk each lane's own runs;
+        // others deal the candidates out, which takes about five times the instructions a candidate.
+        constexpr uint32_t kDealOver = 4;
+        const uint32_t nmax = wave_max(n);
+        if (nmax <= kDealOver * ((T + kWave - 1u) / kWave)) {
             // Four of the lane's candidates per trip: their positions first, then their reads
-            // side by side, then the tests of hash_pairs_of (different bodies, contype /
-            // conaffinity, and the distance unless a plane takes part; the distance is evaluated
-            // whatever the other conditions give and combined with them after).
+            // side by side, then the tests of hash_pairs_of. The walk is bound by VALU issue (two
+            // waves on a SIMD, about 70 instructions a candidate before, some 25 now): candidate
+            // q's position is q plus an offset selected by the run that holds q, without a branch,
+            // with two runs where those at z + 1 are empty in the whole wave; the distance comes
+            // first, and the other conditions are read and tested only where it passes (about 100
+            // of the 601-geom pile's 9,000 candidates a substep). 2048 such piles, four substeps
+            // and the poses to host memory: 1447 -> 1375 us a pass.
             constexpr int U = 4;
-            uint32_t k = 0, left = rl[0], pos = rs[0];
-            for (uint32_t q = 0; q < nmax; q += U) {
-                uint32_t p[U];
-                bool ok[U];
+            const uint32_t e0 = rl[0], e1 = e0 + rl[1], e2 = e1 + rl[2], e3 = e2 + rl[3];
+            auto walk = [&](auto five) {
+                for (uint32_t q = 0; q < nmax; q += U) {
+                    uint32_t o[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    ok[u] = q + (uint32_t)u < n;
-                    p[u] = 0u;
-                    if (ok[u]) {
-                        while (left == 0u) {
-                            ++k;
-                            left = k == 1 ? rl[1] : k == 2 ? rl[2] : k == 3 ? rl[3] : rl[4];
-                            pos = k == 1 ? rs[1] : k == 2 ? rs[2] : k == 3 ? rs[3] : rs[4];
+                    for (int u = 0; u < U; ++u) {
+                        const uint32_t c = q + (uint32_t)u;
+                        uint32_t at = c < e0 ? rs[0] : rs[1] - e0;
+                        if constexpr (decltype(five)::value)
+                            at = c < e1 ? at : c < e2 ? rs[2] - e1 : c < e3 ? rs[3] - e2 : rs[4] - e3;
+                        at += c;  // at or past NG only past the lane's last candidate
+                        o[u] = s.hkey[at < NG ? at : NG - 1u] & 0x3FFFu;
+                    }
+                    float4 pb[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) pb[u] = hash_geom_reach<STAGED>(md, s, hmeta, o[u]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const f3 diff = sub(xyz(pb[u]), xyz(pa4));
+                        const float min_dist = pa4.w + pb[u].w + 0.1f;
+                        if (q + (uint32_t)u < n && !(dot(diff, diff) >= min_dist * min_dist)) {
+                            const uint32_t wb = hash_geom_meta<STAGED>(md, hmeta, o[u]);
+                            hits += hw_body(wb) != hw_body(wa) && hash_filter_pass(a, md, fa, o[u], wb) ? 1u : 0u;
                         }
-                        p[u] = pos;
-                        ++pos;
-                        --left;
                     }
                 }
-                uint32_t o[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) o[u] = s.hkey[p[u]] & 0x3FFFu;
-                uint32_t wb[U];
-                float4 pb[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    wb[u] = hash_geom_meta<STAGED>(md, hmeta, o[u]);
-                    pb[u] = hash_geom_pos<STAGED>(md, s, o[u]);
-                }
-                bool fp[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) fp[u] = hash_filter_pass(a, md, fa, o[u], wb[u]);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const bool pass = hw_body(wb[u]) != hw_body(wa) && fp[u];
-                    const f3 diff = sub(xyz(pb[u]), xyz(pa4));
-                    const float min_dist = pa4.w + pb[u].w + 0.1f;
-                    const bool near = !(dot(diff, diff) >= min_dist * min_dist);
-                    const bool plane = hw_plane(wa) || hw_plane(wb[u]);
-                    hits += (ok[u] && pass && (plane || near)) ? 1u : 0u;
-                }
-            }
+            };
+            if (__ballot(n > e1) != 0ull) walk(std::true_type{});
+            else walk(std::false_type{});
             continue;
         }
         // Four candidates per lane and trip (t, t + 64, t + 128, t + 192), each stage of the
@@ -1163,8 +1179,7 @@ __device__ __forceinline__ uint32_t hash_count_forward(const StepArgs& a, const 
             }
         }
     }
-    for (int d = 1; d < kWave; d <<= 1) hits += (uint32_t)__shfl_xor((int)hits, d);
-    return hits;
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(hits), kWave - 1);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2065,8 +2080,9 @@ void step_kernel(StepArgs a) {
                         const f3 p = add(xyz(s.pos[gr.type_body[1]]), mk3(gr.pos_size0[0], gr.pos_size0[1], gr.pos_size0[2]));
                         const uint32_t id = hash_axis(p.x) + hash_axis(p.y) * 64u + hash_axis(p.z) * 4096u;
                         if (HBM) {
-                            s.hpos[g] = tof4(p, gr.pos_size0[3]);
-                            hmeta[g] = md.hmeta[g];
+                            const uint32_t w = md.hmeta[g];
+                            s.hpos[g] = tof4(p, hw_plane(w) ? __builtin_nanf("") : gr.pos_size0[3]);  // hash_geom_reach
+                            hmeta[g] = w;
                         }
                         a.cell_ids[(size_t)env * a.G + g] = id;
                         key = (id << 14) | g;
