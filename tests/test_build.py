@@ -30,7 +30,7 @@ def test_one_environment_shapes_keep_two_waves_per_simd():
     latency-bound and need two waves per SIMD; above 256 registers the pile's step takes
     2.7x as long."""
     occ = step_occupancy(Path(RESOURCES).read_text())
-    assert occ.get("1,1,0") == 2 and occ.get("1,0,0") == 2 and occ.get("1,2,0") == 2, occ
+    assert all(occ.get(shape, 0) >= 2 for shape in ("1,1,0", "1,0,0", "1,2,0")), occ
 
 
 @pytest.mark.skipif(not Path(RESOURCES).exists(), reason="library not built here")
