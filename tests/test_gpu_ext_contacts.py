@@ -69,3 +69,23 @@ def test_extended_mode_switches_to_the_grouped_shape_and_back():
         g.step(acts[k])
         o.step(acts[k])
         compare(gpu_arrays(g), oracle_arrays(o), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("envs,M", [(40, 200), (1300, 200), (1300, 128)])
+def test_extended_mode_shape_follows_the_env_count(envs, M):
+    """The extended mode's shape, with the model records in LDS for few environments and in HBM
+    where that lets more be resident: each stays on the oracle, and turning the mode off restores
+    the creation-time shape."""
+    g, o, acts = make_pair("pile", envs, 4, seed=9, max_contacts=M)
+    base = (g.modes()["placement"], g.launch_config(), g.waves_per_group(), g.split_groups())
+    g.set_extended_contacts(True)
+    o.extended_contacts = True
+    assert g.launch_config()[0] == 1 and not g.split_groups()
+    for k in range(4):
+        if k == 3:
+            g.set_extended_contacts(False)
+            o.extended_contacts = False
+            assert (g.modes()["placement"], g.launch_config(), g.waves_per_group(), g.split_groups()) == base
+        g.step(acts[k])
+        o.step(acts[k])
+        compare(gpu_arrays(g), oracle_arrays(o), rtol=1e-4, atol=1e-4)

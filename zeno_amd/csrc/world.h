@@ -37,6 +37,7 @@ struct World {
     // The launch shape chosen at creation (extended-contact mode may switch to another one),
     // whether a ZENO_AMD_* variable forced it, and the device's CU count.
     int base_epw = 1, base_waves = 1;
+    uint32_t base_placement = 0;
     bool base_split = false, shape_forced = false;
     int cus = 256;
     EnvLds lds{};

@@ -317,6 +317,7 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     w->epw = epw;
     w->waves = best->waves;
     w->split = best->split;
+    w->base_placement = w->placement;
     w->base_epw = w->epw;
     w->base_waves = w->waves;
     w->base_split = w->split;
@@ -567,14 +568,22 @@ hipError_t World::step(const float* actions, uint32_t substeps, bool actions_on_
     return refresh_views();
 }
 
-// Pool sizes offered to the launch shapes, largest first: the whole list, then fewer slots.
+// Pool sizes offered to the launch shapes, largest first: the whole list, then fewer slots, down to
+// kPoolFloor or a slot per body. Lists past 64 slots that hold fewer than five copies of every
+// body's plane pair keep a pool of the whole list: settled extended piles fill more than 1.5 slots
+// per body of 128, 200 and 256, and a pool that overflows costs more than the environments it lets
+// in (62 bodies, 200 slots, 2053 environments: 561 us a pass with 96 slots, 260 without a pool). Of
+// longer lists few slots are valid, as so many copies of a contact throw the bodies off the ground
+// (64 bodies, 384 and 512 slots: 664 -> 409 and 1612 -> 506 us with the small pool), and the 64-slot
+// lists of robots and piles run faster with it too (40 bodies, 6000 environments: 439 -> 266 us).
 // ZENO_AMD_POOL=n (tests of pools that overflow) offers n alone.
 std::vector<uint32_t> World::pool_sizes() const {
     if (const char* env = std::getenv("ZENO_AMD_POOL")) {
         const int n = std::atoi(env);
         if (n > 0) return {std::min((uint32_t)n, std::max<uint32_t>(M, 1))};
     }
-    const uint32_t m = std::max<uint32_t>(M, 1), floor = std::min(m, std::max(kPoolFloor, (B + 7u) & ~7u));
+    const uint32_t m = std::max<uint32_t>(M, 1), per = M > 64u && M < 5u * B ? M : B;
+    const uint32_t floor = std::min(m, std::max(kPoolFloor, (per + 7u) & ~7u));
     std::vector<uint32_t> sizes{m};
     for (uint32_t c : {512u, 256u, 192u, 128u, 96u, 64u, 48u, 32u, 24u}) {
         if (c < m && c >= floor) sizes.push_back(c);
@@ -586,32 +595,41 @@ std::vector<uint32_t> World::pool_sizes() const {
 void World::set_extended_contacts(bool on) {
     release_graph();
     ext_contacts = on;
-    if (shape_forced || placement != PL_LDS || hash) return;
+    if (shape_forced || base_placement != PL_LDS || hash) return;
+    placement = base_placement;
     epw = base_epw;
     waves = base_waves;
     split = base_split;
     lds = base_lds;
     if (!on || M < 64) return;
     // The grouped narrow phase runs in the one-environment-per-wave instances without split
-    // groups: the best of those by resident environments (the creation-time score).
+    // groups: the best of those by resident environments (the creation-time score), with the
+    // model records in LDS or, where that lets more be resident, in HBM (62 bodies, 200 slots, 2053
+    // environments, two substeps: 213 us with four environments on a CU beside 29 KB of records,
+    // 167 with seven and the records in HBM).
     uint64_t best = 0;
-    for (int w : {4, 1, 2}) {
-        for (uint32_t cap : pool_sizes()) {
-            const EnvLds l = make_env_pool(B, Jp, N, M, cap, false, model.num_geoms, 0, false, false, obsp);
-            const size_t shmem = (size_t)ml.bytes + (size_t)l.bytes * (size_t)w;
-            if (shmem > max_lds_per_workgroup(device)) continue;
-            const int n = resident_workgroups(1, PL_LDS, false, shmem, w, false);
-            if (n <= 0) continue;
-            const uint64_t score = std::min<uint64_t>(E, (uint64_t)n * (uint64_t)w * (uint64_t)cus);
-            if (score > best) {
-                best = score;
-                epw = 1;
-                waves = w;
-                split = false;
-                lds = l;
-            }
+    auto offer = [&](uint32_t pl, int w, uint32_t cap) {
+        const bool own = pl == PL_MODEL_HBM;
+        const EnvLds l = make_env_pool(B, Jp, N, M, cap, false, model.num_geoms, own ? 16 * kJRecQuads * nrec : 0, own,
+                                       own && sweep_n != 0, obsp);
+        const size_t shmem = (own ? (size_t)0 : (size_t)ml.bytes) + (size_t)l.bytes * (size_t)w;
+        if (shmem > max_lds_per_workgroup(device)) return;
+        const int n = resident_workgroups(1, pl, false, shmem, w, false);
+        if (n <= 0) return;
+        const uint64_t score = std::min<uint64_t>(E, (uint64_t)n * (uint64_t)w * (uint64_t)cus);
+        if (score > best) {
+            best = score;
+            placement = pl;
+            epw = 1;
+            waves = w;
+            split = false;
+            lds = l;
         }
+    };
+    for (int w : {4, 1, 2}) {
+        for (uint32_t cap : pool_sizes()) offer(PL_LDS, w, cap);
     }
+    for (uint32_t cap : pool_sizes()) offer(PL_MODEL_HBM, 1, cap);
 }
 
 void World::release_graph() {
