@@ -3063,12 +3063,7 @@ void step_kernel(StepArgs a) {
         if constexpr (POOL) {
             if (hv.contacts) {
                 wave_sync<true>();
-                // A quad per lane: each store covers whole 64-B lines of host memory (a record per
-                // lane writes a quarter of 4 G lines at a time).
-                const float4* from = (const float4*)list;
-                float4* const to = (float4*)(hv.contacts + (size_t)env * M);
-#pragma unroll 4
-                for (uint32_t q = sl; q < 4 * n_out; q += G) to[q] = from[q];
+                for (uint32_t k = sl; k < n_out; k += G) copy_record(&hv.contacts[(size_t)env * M + k], &list[k]);
             }
         } else
         for (uint32_t k = sl; k < n_out; k += G) {
