@@ -47,7 +47,11 @@ struct World {
     bool hrows = false;  // hash filter classes fit the model's rows (build_hash_words)
     uint32_t placement = PL_LDS;  // where the step kernel keeps model records and working sets
     bool ext_contacts = false;    // extended-contact mode (zeno_amd_world_set_extended_contacts)
-    bool resort = false;          // counts set by the host: the next launch sorts unconditionally
+    // Counts set by the host: the next launch that advances an environment sorts its list
+    // unconditionally. Set until every environment has advanced; `sorted_since` marks those that
+    // have, where only some did (empty: none).
+    bool resort = false;
+    std::vector<uint8_t> sorted_since;
     hipStream_t stream = nullptr;
     size_t device_bytes = 0;
 
@@ -120,7 +124,8 @@ struct World {
     // arguments are those of capture time, so the setters that change them release it.
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    uint32_t graph_steps = 0;
+    struct Schedule { const float* d_act; uint64_t stride_bytes; uint32_t steps, substeps; };
+    Schedule schedule{};  // what the graph runs
     static constexpr uint32_t kFusedCalls = 64;  // steps per captured launch
     bool capturing = false;
 
@@ -155,6 +160,7 @@ struct World {
    private:
     std::vector<uint32_t> pool_sizes() const;
     hipError_t launch(const float* d_act, uint32_t substeps, const uint8_t* d_step_mask, uint32_t calls = 1, uint64_t action_stride = 0);
+    hipError_t enqueue_schedule();
     hipError_t stage_actions(const float* actions, const float** d_out);
     hipError_t mark_actions_used();
     hipError_t upload_mask(const uint8_t* mask, uint8_t** d_out);

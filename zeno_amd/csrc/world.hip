@@ -451,11 +451,10 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
     a.hrows = hrows ? 1u : 0u;
     a.cell_ids = d_cell_ids;
     a.ext_contacts = ext_contacts ? 1u : 0u;
-    a.sort_all = resort ? 1u : 0u;
+    a.sort_all = resort && !capturing ? 1u : 0u;  // a captured launch runs later, or never
     a.sweep = d_sweep; a.sweep_n = sweep_n; a.sweep_planes = sweep_planes;
     // Only where it saves a pass: the bodies after body 0 fill whole passes of the lanes.
     a.b_first = (b0_static && (B - 1u) % (64u / (uint32_t)epw) == 0u) ? 1u : 0u;
-    resort = false;
     a.placement = placement;
     a.work = d_work;
     a.iters = iters; a.substeps = substeps;
@@ -564,6 +563,7 @@ hipError_t World::step(const float* actions, uint32_t substeps, bool actions_on_
     if (actions_on_device) d_act = actions;
     else if (A > 0) { ZA_TRY(stage_actions(actions, &d_act)); staged = true; }
     ZA_TRY(launch(d_act, actual, nullptr));
+    resort = false;
     if (staged) ZA_TRY(mark_actions_used());
     return refresh_views();
 }
@@ -639,7 +639,6 @@ void World::release_graph() {
     if (graph) hipGraphDestroy(graph);
     graph_exec = nullptr;
     graph = nullptr;
-    graph_steps = 0;
 }
 
 // `steps` consecutive steps, step k reading its actions at d_actions + k * stride_bytes,
@@ -655,16 +654,10 @@ hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint3
     ZA_TRY(hipSetDevice(device));
     release_graph();
     ZA_TRY(hipStreamSynchronize(stream));
-    const uint32_t actual = substeps == 0 ? adaptive_substeps : substeps;
-    dt = timestep / (float)std::max<uint32_t>(actual, 1);
+    schedule = Schedule{d_act, stride_bytes, steps, substeps == 0 ? adaptive_substeps : substeps};
     ZA_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     capturing = true;
-    hipError_t e = hipSuccess;
-    for (uint32_t k = 0; k < steps && e == hipSuccess; k += kFusedCalls) {
-        const float* a = A > 0 ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(d_act) + k * stride_bytes)
-                               : d_actions;
-        e = launch(a, actual, nullptr, std::min(kFusedCalls, steps - k), A > 0 ? stride_bytes : 0);
-    }
+    hipError_t e = enqueue_schedule();
     capturing = false;
     hipGraph_t g = nullptr;
     const hipError_t ec = hipStreamEndCapture(stream, &g);
@@ -677,13 +670,30 @@ hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint3
         return e;
     }
     graph = g;
-    graph_steps = steps;
+    return hipSuccess;
+}
+
+hipError_t World::enqueue_schedule() {
+    const Schedule& c = schedule;
+    dt = timestep / (float)std::max<uint32_t>(c.substeps, 1);
+    for (uint32_t k = 0; k < c.steps; k += kFusedCalls) {
+        const float* a = A > 0 ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(c.d_act) + k * c.stride_bytes)
+                               : d_actions;
+        ZA_TRY(launch(a, c.substeps, nullptr, std::min(kFusedCalls, c.steps - k), A > 0 ? c.stride_bytes : 0));
+    }
     return hipSuccess;
 }
 
 hipError_t World::graph_launch() {
     if (!graph_exec) return hipErrorInvalidValue;
     ZA_TRY(hipSetDevice(device));
+    // Counts set since the last step: the schedule's launches run as they are, with the sort that
+    // the captured ones do without (each sorts; what is in order stays as it is).
+    if (resort) {
+        ZA_TRY(enqueue_schedule());
+        resort = false;
+        return refresh_views();
+    }
     ZA_TRY(hipGraphLaunch(graph_exec, stream));
     mark_all_dirty();
     return refresh_views();
@@ -728,6 +738,16 @@ hipError_t World::step_subset(const float* actions, const uint8_t* mask, uint32_
     uint8_t* dm = nullptr;
     ZA_TRY(upload_mask(mask, &dm));
     ZA_TRY(launch(d_act, actual, dm));
+    if (resort) {
+        // The environments held back keep their unsorted lists.
+        if (sorted_since.empty()) sorted_since.assign(E, 0);
+        uint32_t left = 0;
+        for (uint32_t e = 0; e < E; ++e) {
+            sorted_since[e] |= mask[e] ? 1 : 0;
+            left += sorted_since[e] ? 0u : 1u;
+        }
+        resort = left != 0u;
+    }
     if (staged) ZA_TRY(mark_actions_used());
     return refresh_views();
 }
@@ -756,6 +776,7 @@ hipError_t World::set_contact_counts(const uint32_t* counts) {
     ZA_TRY(hipMemcpyAsync(d_counts, counts, (size_t)E * 4, hipMemcpyHostToDevice, stream));
     ZA_TRY(hipStreamSynchronize(stream));
     resort = true;  // the next step sorts every env's first min(count, M) slots
+    sorted_since.clear();
     mark_all_dirty();
     return refresh_views();
 }
