@@ -89,3 +89,41 @@ def test_extended_mode_shape_follows_the_env_count(envs, M):
         g.step(acts[k])
         o.step(acts[k])
         compare(gpu_arrays(g), oracle_arrays(o), rtol=1e-4, atol=1e-4)
+
+
+def negative_radii_mjcf(bodies: int = 6) -> str:
+    geoms = ('<geom type="sphere" size="-0.3" mass="1"/>', '<geom type="box" size="0.2 0.15 0.1" mass="1"/>',
+             '<geom type="capsule" size="-0.25 0.1" mass="1"/>')
+    rows = [f'<body name="b{i}" pos="{0.1 * i:.3f} {0.05 * (i % 2):.3f} {0.4 + 0.05 * i:.3f}"><joint type="free"/>{geoms[i % 3]}</body>'
+            for i in range(bodies)]
+    return '<mujoco><worldbody><geom type="plane" size="20 20 0.1"/>' + "".join(rows) + "</worldbody></mujoco>"
+
+
+@pytest.mark.parametrize("M", [48, 64, 200])
+def test_hits_of_negative_penetration(M):
+    """A sphere or capsule of negative radius takes part in hits whose penetration is negative:
+    their slots get the point, normal and friction, and neither the matching nor the solve visits
+    them."""
+    from oracle.oracle import OracleWorld
+    from zeno_amd.model import load_model
+    from zeno_amd.world import ZenoWorld
+
+    xml = negative_radii_mjcf()
+    g = ZenoWorld(mjcf_string=xml, num_envs=3, max_contacts_per_env=M)
+    o = OracleWorld(load_model(mjcf_string=xml), 3, max_contacts_per_env=M)
+    g.set_extended_contacts(True)
+    o.extended_contacts = True
+    rng = np.random.default_rng(2)
+    state = [x.copy() for x in (o.positions, o.quaternions, o.velocities, o.angular_velocities)]
+    state[2][:, 1:, :3] = rng.uniform(-2, 2, (3, 6, 3))
+    state[3][:, 1:, :3] = rng.uniform(-3, 3, (3, 6, 3))
+    for w in (g, o):
+        w.reset_to_state(*state)
+    none, seen = np.zeros((3, 0), np.float32), 0
+    for k in range(8):
+        g.step(none)
+        o.step(none)
+        pen = o.contacts["position_pen"][..., 3]
+        seen += int(((pen < 0) & (pen != -1)).sum())
+        compare(gpu_arrays(g), oracle_arrays(o), 0.0, 0.0)
+    assert seen > 0

@@ -232,7 +232,14 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     // pool is taken only where it lets more environments be resident (the score below), and none
     // below kPoolFloor slots or one per body, since a substep with more valid slots than the pool
     // holds runs its contact solve out of HBM.
-    const std::vector<uint32_t> caps = w->hash ? std::vector<uint32_t>{0u} : w->M > kPoolMaxList ? std::vector<uint32_t>{} : w->pool_sizes();
+    // A sphere or capsule of negative radius can be in contact at a negative penetration in the
+    // extended-contact mode: such a slot is recorded but not solved, where a pool solves all that it
+    // holds, so these models keep their list in the working set (placements 2 and 3).
+    const bool negative_radius = std::any_of(m.geoms.begin(), m.geoms.end(), [](const GeomRec& g) {
+        return (g.type_body[0] == GEOM_SPHERE || g.type_body[0] == GEOM_CAPSULE) && g.pos_size0[3] < 0.0f;
+    });
+    const std::vector<uint32_t> caps = w->hash ? std::vector<uint32_t>{0u}
+                                     : w->M > kPoolMaxList || negative_radius ? std::vector<uint32_t>{} : w->pool_sizes();
     auto pool = [&](uint32_t cap, bool split, bool own) {
         return make_env_pool(w->B, w->Jp, w->N, std::max<uint32_t>(w->M, 1), cap, split, m.num_geoms,
                              own ? 16 * kJRecQuads * w->nrec : 0, own, w->sweep_n != 0, w->obsp);
