@@ -88,6 +88,18 @@ def _cases():
 
 CASES = _cases()
 
+# Solved by one lane, each on a moved anchor: between two free bodies a limited slide past its
+# upper end, and a weld.
+SINGLE_LANE = """<mujoco><worldbody>
+  <body name="a" pos="0 0 2"><joint type="free"/><geom type="sphere" size="0.1" mass="1"/>
+    <body name="b" pos="0.3 0.1 0.2"><joint type="slide" axis="1 2 0.5" pos="0.05 -0.1 0.07" limited="true" range="-0.05 0.05"/>
+      <geom type="sphere" size="0.1" mass="0.5"/></body>
+    <body name="c" pos="-0.3 0.2 0.1" quat="0.9 0.1 0.3 0.2"><geom type="sphere" size="0.1" mass="0.7"/></body>
+  </body></worldbody></mujoco>"""
+MOVED = {1: dict(quat=P._qaxis([0, 0, 1], 0.3), vel=(0.2, -0.1, 0.05), angvel=(0.5, 0, 0)),
+         2: dict(pos=(0.5, 0.4, 2.25), quat=P._qaxis([1, 2, 3], 0.2)), 3: dict(pos=(-0.2, 0.25, 2.0))}
+CASES["single_lane_joints"] = (SINGLE_LANE, (0, 0, 0), 4, 1, MOVED, None)
+
 
 def _state(w_like, B, setup):
     """[E, B, 4] arrays from the model's initial state with `setup` applied to every env; env k
@@ -127,3 +139,12 @@ def test_pin_scene_matches_oracle(name):
         o.step(acts[:, : m["num_actuators"]] if m["num_actuators"] else None)
         compare(gpu_arrays(g), oracle_arrays(o), rtol=1e-5, atol=1e-6)
     g.close()
+
+
+@pytest.mark.parametrize("placement", ["1", "2", "3"])
+@pytest.mark.parametrize("name", ["single_lane_joints", "slider_rotated", "weld_rotated", "weld_dynamic_parent", "slide_state_solved"])
+def test_single_lane_joints_in_every_placement(monkeypatch, name, placement):
+    """Weld, slider and linear-limit records (no lane-pair header, anchors in the second half) with
+    the bodies in LDS and in HBM."""
+    monkeypatch.setenv("ZENO_AMD_PLACEMENT", placement)
+    test_pin_scene_matches_oracle(name)

@@ -235,10 +235,10 @@ __device__ __forceinline__ q4 qdelta_signed(f3 d, q4 q, float sg) { return qscal
 struct JHalf { float4 h0, mi, v1, v2; };
 __device__ __forceinline__ JHalf load_half(const float4* p) { return JHalf{p[0], p[1], p[2], p[3]}; }
 // The state a lane-pair solve reads for the lane's body: position, orientation and the
-// constraint's multiplier (every record's header holds a valid multiplier index).
+// constraint's multiplier.
 struct JState { float4 P, Q; float lam; };
 // The header's x is the byte offset of the lane's body in the body arrays and its z the
-// multiplier's (fill_alpha).
+// multiplier's (fill_alpha, in the lane-pair types' records alone).
 template <int BS>
 __device__ __forceinline__ float4* jbody(const BodyArr<BS>& arr, const JHalf& h) {
     return (float4*)((unsigned char*)arr.p + fbits(h.h0.x));
@@ -774,16 +774,16 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
     }
 }
 
-// One joint solve of the given type on the lane pair: h is the lane's half record and st its
-// body's state (lane-pair types), r the whole record in LDS (single-lane types, run by body
-// a's lane, which read the state themselves).
+// One joint solve of the given type on the lane pair: h is the lane's half record (lane-pair
+// types), r the whole record in LDS (single-lane types, run by body a's lane). The body's state is
+// read once the type is known: of a single-lane record only the first half starts with a header,
+// and its fields are indices, not byte offsets.
 template <int BS>
-__device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const JState& st, const float4* r,
-                                            const LdsT<BS>& s, bool odd) {
+__device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const float4* r, const LdsT<BS>& s, bool odd) {
     switch (type) {
-        case C_POSITIONAL: solve_positional2(h, st, s, odd, com); break;
-        case C_ANGULAR: solve_angular2(h, st, s, odd); break;
-        case C_ANGULAR_LIMIT: solve_angular_limit2(h, st, s, odd); break;
+        case C_POSITIONAL: solve_positional2(h, load_jstate(h, s), s, odd, com); break;
+        case C_ANGULAR: solve_angular2(h, load_jstate(h, s), s, odd); break;
+        case C_ANGULAR_LIMIT: solve_angular_limit2(h, load_jstate(h, s), s, odd); break;
         case C_WELD: if (!odd) solve_weld(r, s); break;
         case C_LINEAR_LIMIT: if (!odd) solve_linear_limit(r, s); break;
         case C_SLIDER: if (!odd) solve_slider(r, s); break;
@@ -2833,12 +2833,11 @@ void step_kernel(StepArgs a) {
                     const uint32_t st = __builtin_amdgcn_readfirstlane(ph1.start), cn = __builtin_amdgcn_readfirstlane(ph1.count);
                     nxt = load_half(md.jrec + (st + (kf < cn ? kf : 0u)) * kJRecQuads + half);
                 }
-                if (live && kf < cnt) solve_joint(type, com, cur, load_jstate(cur, s), md.jrec + (start + kf) * kJRecQuads, s, odd);
+                if (live && kf < cnt) solve_joint(type, com, cur, md.jrec + (start + kf) * kJRecQuads, s, odd);
                 if (live) {
                     for (uint32_t k = kf + G / 2; k < cnt; k += G / 2) {
                         const float4* r = md.jrec + (start + k) * kJRecQuads;
-                        const JHalf hk = load_half(r + half);
-                        solve_joint(type, com, hk, load_jstate(hk, s), r, s, odd);
+                        solve_joint(type, com, load_half(r + half), r, s, odd);
                     }
                 }
                 wave_sync<HBM>();
