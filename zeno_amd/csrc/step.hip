@@ -234,9 +234,6 @@ __device__ __forceinline__ q4 qdelta_signed(f3 d, q4 q, float sg) { return qscal
 // and its centre of mass or the angular limits.
 struct JHalf { float4 h0, mi, v1, v2; };
 __device__ __forceinline__ JHalf load_half(const float4* p) { return JHalf{p[0], p[1], p[2], p[3]}; }
-// The state a lane-pair solve reads for the lane's body: position, orientation and the
-// constraint's multiplier.
-struct JState { float4 P, Q; float lam; };
 // The header's x is the byte offset of the lane's body in the body arrays and its z the
 // multiplier's (fill_alpha, in the lane-pair types' records alone).
 template <int BS>
@@ -247,11 +244,6 @@ template <int BS>
 __device__ __forceinline__ float* jlam(const LdsT<BS>& s, const JHalf& h) {
     return (float*)((unsigned char*)s.lam + fbits(h.h0.z));
 }
-template <int BS>
-__device__ __forceinline__ JState load_jstate(const JHalf& h, const LdsT<BS>& s) {
-    return JState{*jbody(s.pos, h), *jbody(s.quat, h), *jlam(s, h)};
-}
-
 // Late selects. The positional and hinge solves evaluate their update unconditionally and
 // apply the reference's conditions (C > 1e-6, w > 1e-8, inverse mass > 0) only to the values
 // they store: a compare that feeds a branch or a select right away waits about 30 cycles for
@@ -268,14 +260,14 @@ __device__ __forceinline__ JState load_jstate(const JHalf& h, const LdsT<BS>& s)
 // and a normalised quaternion has components within [-1, 1] or is the identity. Phases without
 // such a body, most of every robot's, skip the rotation (33 of about 300 instructions).
 template <int BS>
-__device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd, bool com) {
+__device__ __forceinline__ void solve_positional2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd, bool com) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
     const float sg = odd ? -1.0f : 1.0f;
-    const f3 P = xyz(st.P);
-    const q4 Q = toq(st.Q);
-    const float lambda_prev = st.lam;
+    const f3 P = xyz(*jbody(s.pos, h));
+    const q4 Q = toq(quat);
+    const float lambda_prev = *jlam(s, h);
     const f3 rr = qrot_fixed(xyz(h.v1), Q);                // r_a or r_b
     const f3 u = add(P, rr);                               // pos + r
     const f3 diff = sub(pair_a(u), pair_b(u));             // (pos_a + r_a) - (pos_b + r_b)
@@ -298,11 +290,11 @@ __device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& 
 
 // :1131-1186 hinge axis alignment, lane pair.
 template <int BS>
-__device__ __forceinline__ void solve_angular2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
+__device__ __forceinline__ void solve_angular2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
-    const q4 Q = toq(st.Q);
+    const q4 Q = toq(quat);
     const f3 axw = qrot_fixed(xyz(h.v1), Q);
     const f3 cr = cross(pair_a(axw), pair_b(axw));
     const float sin_angle = len_gate(cr);
@@ -319,14 +311,14 @@ __device__ __forceinline__ void solve_angular2(const JHalf& h, const JState& st,
 
 // :1189-1238 angular limit, lane pair.
 template <int BS>
-__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
+__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
     const float sg = odd ? -1.0f : 1.0f;
     const f3 axis_local = xyz(h.v1);
     const float lower = h.v2.x, upper = h.v2.y;
-    const q4 Q = toq(st.Q);
+    const q4 Q = toq(quat);
     const q4 qa = pair_a(Q), qb = pair_b(Q);
     const q4 q_rel = qmul(qconj(qa), qb);
     const float angle = 2.0f * z_atan2f(dot(xyz(q_rel), axis_local), q_rel.w);
@@ -776,14 +768,19 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
 
 // One joint solve of the given type on the lane pair: h is the lane's half record (lane-pair
 // types), r the whole record in LDS (single-lane types, run by body a's lane). The body's state is
-// read once the type is known: of a single-lane record only the first half starts with a header,
-// and its fields are indices, not byte offsets.
+// read for the lane-pair types alone: of a single-lane record only the first half starts with a
+// header, and its fields are indices, not byte offsets. The orientation is read before the types
+// are told apart, the position and the multiplier by the one type that uses them.
 template <int BS>
 __device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const float4* r, const LdsT<BS>& s, bool odd) {
+    if (joint_type_paired(type)) {
+        const float4 quat = *jbody(s.quat, h);
+        if (type == C_POSITIONAL) solve_positional2(h, quat, s, odd, com);
+        else if (type == C_ANGULAR) solve_angular2(h, quat, s, odd);
+        else solve_angular_limit2(h, quat, s, odd);
+        return;
+    }
     switch (type) {
-        case C_POSITIONAL: solve_positional2(h, load_jstate(h, s), s, odd, com); break;
-        case C_ANGULAR: solve_angular2(h, load_jstate(h, s), s, odd); break;
-        case C_ANGULAR_LIMIT: solve_angular_limit2(h, load_jstate(h, s), s, odd); break;
         case C_WELD: if (!odd) solve_weld(r, s); break;
         case C_LINEAR_LIMIT: if (!odd) solve_linear_limit(r, s); break;
         case C_SLIDER: if (!odd) solve_slider(r, s); break;
