@@ -21,6 +21,8 @@
 // list is written back.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "dmath.h"
@@ -3121,19 +3123,27 @@ hipError_t allow_lds(size_t shmem) {
     return e;
 }
 
+// Workgroups of `waves` waves resident on a CU: what the registers and the wave slots allow, asked of
+// HIP once per instance and workgroup size, and what the LDS allows. HIP's own answer for a given
+// LDS size divides the 160 KB by the bytes asked for, but a workgroup takes whole kLdsUnits (three
+// workgroups of 54,064 bytes: 3 by HIP's answer, 2 resident).
 template <int EPW, int PL, bool HASH, bool GROUP = false, bool SPLIT = false>
 int resident_as(size_t shmem, int waves = 1) {
-    // A shape that does not fit is an answer here, not an error: the failed query's error
-    // is taken off HIP's last-error slot so that later hipGetLastError checks (of this or
-    // another world) do not report it.
-    int n = 0;
-    if (allow_lds<EPW, PL, HASH, GROUP, SPLIT>(shmem) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, step_kernel<EPW, PL, HASH, GROUP, SPLIT>, kWave * waves, shmem) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
+    constexpr int kUnknown = -1;
+    static std::atomic<int> by_registers[2 * kMaxWaves + 1] = {kUnknown, kUnknown, kUnknown, kUnknown, kUnknown,
+                                                               kUnknown, kUnknown, kUnknown, kUnknown};
+    int n = by_registers[waves].load(std::memory_order_relaxed);
+    if (n == kUnknown) {
+        // A shape that does not fit is an answer here, not an error: the failed query's error
+        // is taken off HIP's last-error slot so that later hipGetLastError checks (of this or
+        // another world) do not report it.
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, step_kernel<EPW, PL, HASH, GROUP, SPLIT>, kWave * waves, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        by_registers[waves].store(n, std::memory_order_relaxed);
     }
-    return n;
+    return (int)std::min<size_t>((size_t)n, lds_workgroups(shmem));
 }
 
 template <int EPW, int PL, bool HASH, bool GROUP = false, bool SPLIT = false>
