@@ -25,3 +25,18 @@ def test_workgroups_that_the_lds_holds(tmp_path):
     rows = run(tmp_path, 'for (size_t b : {53760, 53761, 81920, 81921, 12800, 12801, 163840, 163841, 1, 0})'
                          ' printf("%zu %zu\\n", b, lds_workgroups(b));')
     assert dict(rows) == {53760: 3, 53761: 2, 81920: 2, 81921: 1, 12800: 12, 12801: 11, 163840: 1, 163841: 0, 1: 128, 0: 163840}
+
+
+def test_smallest_pool(tmp_path):
+    """(bodies, free bodies, list) -> slots: robots by their bodies, piles by how many copies of a
+    body's ground contact their list holds, never below the most valid slots seen settled (the last
+    number, with the list's own length as the bound)."""
+    seen = [(13, 12, 64, 22), (13, 12, 128, 21), (25, 24, 64, 59), (25, 24, 80, 58), (25, 24, 128, 33), (25, 24, 200, 24),
+            (39, 38, 64, 62), (39, 38, 80, 76), (39, 38, 128, 90), (39, 38, 200, 56), (39, 38, 256, 35), (41, 40, 200, 48),
+            (51, 50, 128, 100), (51, 50, 200, 96), (51, 50, 256, 68), (51, 50, 384, 26), (63, 62, 128, 108), (63, 62, 200, 115),
+            (63, 62, 256, 120), (63, 62, 384, 69), (63, 62, 512, 30)]
+    rows = run(tmp_path, "\n".join(f'printf("%u\\n", pool_floor({b}, {n}, {m}));' for b, n, m, _ in seen)
+               + 'printf("%u %u %u\\n", pool_floor(14, 0, 64), pool_floor(30, 0, 64), pool_floor(2, 0, 1));')
+    for (b, n, m, most), (slots,) in zip(seen, rows):
+        assert min(slots, m) >= most, (b, n, m, slots, most)
+    assert rows[-1] == [24, 32, 24]

@@ -190,6 +190,12 @@ inline size_t lds_workgroups(size_t bytes) { return bytes == 0 ? kLdsPerCu : kLd
 // filled), then the levels.
 constexpr uint32_t kPoolMaxList = 1536;  // longer lists keep placement 3 (everything in HBM), as documented
 constexpr uint32_t kPoolFloor = 24;    // smallest pool offered (or the list, or one slot per body)
+// Smallest pool offered for lists of M slots: of B bodies, n_free hang on no joint (World::pool_sizes).
+inline uint32_t pool_floor(uint32_t B, uint32_t n_free, uint32_t M) {
+    const uint64_t n = n_free, half_slots = M < 5 * n ? 5 * n : M < 7 * n ? 3 * n : 2 * n;
+    const uint64_t slots = std::max<uint64_t>((half_slots + 1) / 2, B);
+    return (uint32_t)std::max<uint64_t>(kPoolFloor, (slots + 7) / 8 * 8);
+}
 constexpr uint32_t kBodyQuadsSplit = 9, kBodyQuads = 7;
 constexpr uint32_t kPoolClasses = 64;  // ordered geom-type pairs of the grouped narrow phase
 inline EnvLds make_env_pool(uint32_t B, uint32_t Jp, uint32_t N, uint32_t M, uint32_t cap, bool split, uint32_t G = 0,

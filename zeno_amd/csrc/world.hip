@@ -576,21 +576,29 @@ hipError_t World::step(const float* actions, uint32_t substeps, bool actions_on_
 }
 
 // Pool sizes offered to the launch shapes, largest first: the whole list, then fewer slots, down to
-// kPoolFloor or a slot per body. Lists past 64 slots that hold fewer than five copies of every
-// body's plane pair keep a pool of the whole list: settled extended piles fill more than 1.5 slots
-// per body of 128, 200 and 256, and a pool that overflows costs more than the environments it lets
-// in (62 bodies, 200 slots, 2053 environments: 561 us a pass with 96 slots, 260 without a pool). Of
-// longer lists few slots are valid, as so many copies of a contact throw the bodies off the ground
-// (64 bodies, 384 and 512 slots: 664 -> 409 and 1612 -> 506 us with the small pool), and the 64-slot
-// lists of robots and piles run faster with it too (40 bodies, 6000 environments: 439 -> 266 us).
+// a floor that keeps pools from overflowing (a substep with more valid slots than its pool holds
+// solves out of HBM, its whole wave with it: 62 bodies, 256 slots, 3000 environments take 239 us
+// with 96 slots for up to 120 valid ones, 180 with 128, 231 with the whole list).
+// A robot's bodies hang together and few of its slots are valid (at most 27 of 64 over hundreds of
+// steps; 24 slots or the whole list take the same time within 3%, and a pool of one slot, where
+// every contact overflows, 4-15% more): kPoolFloor or a slot per body.
+// A free body can lie on the ground with as many valid slots as the list holds copies of its plane
+// pair. Settled piles of 12 to 62 bodies have had at most 2.4 valid slots per body where the list
+// holds fewer than five per body, 1.5 below seven (38 bodies and 200 slots: 148 us with 40 slots,
+// 118 with 64) and 1 above, where so many copies throw the bodies off the ground; only 12 bodies in
+// lists of 200 and more passed that, in one environment of a hundred at most.
 // ZENO_AMD_POOL=n (tests of pools that overflow) offers n alone.
 std::vector<uint32_t> World::pool_sizes() const {
+    const uint32_t m = std::max<uint32_t>(M, 1);
     if (const char* env = std::getenv("ZENO_AMD_POOL")) {
         const int n = std::atoi(env);
-        if (n > 0) return {std::min((uint32_t)n, std::max<uint32_t>(M, 1))};
+        if (n > 0) return {std::min((uint32_t)n, m)};
     }
-    const uint32_t m = std::max<uint32_t>(M, 1), per = M > 64u && M < 5u * B ? M : B;
-    const uint32_t floor = std::min(m, std::max(kPoolFloor, (per + 7u) & ~7u));
+    std::vector<uint8_t> free_body(B, 1);
+    for (const ConstraintRec& c : model.templates) free_body[c.indices[0]] = free_body[c.indices[1]] = 0;
+    uint32_t n_free = 0;
+    for (uint32_t b = 0; b < B; ++b) n_free += free_body[b] && model.inv_mass_inertia[4 * b] > 0.0f ? 1u : 0u;
+    const uint32_t floor = std::min(m, pool_floor(B, n_free, M));
     std::vector<uint32_t> sizes{m};
     for (uint32_t c : {512u, 256u, 192u, 128u, 96u, 64u, 48u, 32u, 24u}) {
         if (c < m && c >= floor) sizes.push_back(c);
