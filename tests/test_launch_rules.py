@@ -40,3 +40,12 @@ def test_smallest_pool(tmp_path):
     for (b, n, m, most), (slots,) in zip(seen, rows):
         assert min(slots, m) >= most, (b, n, m, slots, most)
     assert rows[-1] == [24, 32, 24]
+
+
+def test_steps_of_a_captured_launch(tmp_path):
+    """Up to 64 substeps or one step, what is left of the schedule, and no product past 32 bits."""
+    cases = [(1, 130), (1, 3), (2, 130), (5, 130), (63, 9), (64, 9), (65, 9), (1 << 26, 64), (0xFFFFFFFF, 64), (0, 70)]
+    rows = run(tmp_path, "\n".join(f'printf("%u\\n", fused_calls({s}u, {left}u));' for s, left in cases))
+    assert [n for n, in rows] == [64, 3, 32, 12, 1, 1, 1, 1, 1, 64]
+    assert all(n * s < 1 << 32 for (n,), (s, _) in zip(rows, cases))
+

@@ -455,6 +455,15 @@ inline ModelLayout make_model_layout(uint32_t B, uint32_t J, uint32_t G, uint32_
     return L;
 }
 
+// Steps (zeno_world_step calls) that one launch of a captured schedule takes: as many as make up
+// kFusedSubsteps, at least one. The bound is on substeps, so that a launch's time is at most that of
+// kFusedSubsteps eager one-substep steps, or of one eager step, whatever the scene; it also keeps
+// calls * substeps within 32 bits.
+constexpr uint32_t kFusedSubsteps = 64;
+inline uint32_t fused_calls(uint32_t substeps, uint32_t steps_left) {
+    return std::min(steps_left, std::max(1u, kFusedSubsteps / std::max(substeps, 1u)));
+}
+
 struct StepArgs {
     // Sizes. G = geoms; Gp = G rounded up to a power of two (hash mode).
     uint32_t E, B, J, Jp, A, S, obsp, N, nrec, njph, M, P, G, Gp;

@@ -126,7 +126,6 @@ struct World {
     hipGraphExec_t graph_exec = nullptr;
     struct Schedule { const float* d_act; uint64_t stride_bytes; uint32_t steps, substeps; };
     Schedule schedule{};  // what the graph runs
-    static constexpr uint32_t kFusedCalls = 64;  // steps per captured launch
     bool capturing = false;
 
     ~World();

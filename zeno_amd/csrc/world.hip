@@ -658,11 +658,10 @@ void World::release_graph() {
 
 // `steps` consecutive steps, step k reading its actions at d_actions + k * stride_bytes,
 // captured from the world's stream into one HIP graph: a replay is one launch call for the
-// whole sequence. Environments do not meet within a step, so a launch takes kFusedCalls steps
+// whole sequence. Environments do not meet within a step, so a launch takes fused_calls() steps
 // one after another without storing and reloading the state between them, and an environment
-// with many contacts in one step holds no other up: a node per kFusedCalls steps instead of per
-// step (Ant, 4096 environments, 32 steps: 2041 -> 1370 us; the bound keeps a launch of the
-// slowest scenes well under a second). Every node is a step-kernel launch (no memset or copy
+// with many contacts in one step holds no other up: a node for up to 64 steps instead of one per
+// step (Ant, 4096 environments, 32 steps: 2041 -> 1370 us). Every node is a step-kernel launch (no memset or copy
 // nodes). Substeps, dt, gravity, the contact mode and the buffer addresses are fixed at
 // capture; the world's setters for them release the graph.
 hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint32_t steps, uint32_t substeps) {
@@ -691,10 +690,11 @@ hipError_t World::capture_steps(const float* d_act, uint64_t stride_bytes, uint3
 hipError_t World::enqueue_schedule() {
     const Schedule& c = schedule;
     dt = timestep / (float)std::max<uint32_t>(c.substeps, 1);
-    for (uint32_t k = 0; k < c.steps; k += kFusedCalls) {
+    for (uint32_t k = 0, n = 0; k < c.steps; k += n) {
+        n = fused_calls(c.substeps, c.steps - k);
         const float* a = A > 0 ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(c.d_act) + k * c.stride_bytes)
                                : d_actions;
-        ZA_TRY(launch(a, c.substeps, nullptr, std::min(kFusedCalls, c.steps - k), A > 0 ? c.stride_bytes : 0));
+        ZA_TRY(launch(a, c.substeps, nullptr, n, A > 0 ? c.stride_bytes : 0));
     }
     return hipSuccess;
 }
