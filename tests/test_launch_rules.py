@@ -49,3 +49,28 @@ def test_steps_of_a_captured_launch(tmp_path):
     assert [n for n, in rows] == [64, 3, 32, 12, 1, 1, 1, 1, 1, 64]
     assert all(n * s < 1 << 32 for (n,), (s, _) in zip(rows, cases))
 
+
+def test_every_joint_record_has_both_headers(tmp_path):
+    """The lanes of a pair form their addresses from the half records' headers before the type is
+    told apart: bodies, multiplier and type stand in both halves, whatever the type, and the second
+    anchor keeps out of them."""
+    rows = run(tmp_path, """
+    const uint32_t types[] = {C_POSITIONAL, C_WELD, C_ANGULAR, C_ANGULAR_LIMIT, C_LINEAR_LIMIT, C_SLIDER};
+    std::vector<ConstraintRec> t(6);
+    std::vector<uint32_t> ranges;
+    for (uint32_t k = 0; k < 6; ++k) {
+        t[k] = ConstraintRec{};
+        t[k].indices[0] = 2 * k + 1; t[k].indices[1] = 2 * k + 2; t[k].indices[3] = types[k];
+        t[k].anchor_b[0] = 0.25f; t[k].anchor_b[1] = 100.0f; t[k].anchor_b[2] = -3.0f;
+        t[k].limits[0] = -0.1f; t[k].limits[1] = 0.1f;
+        ranges.push_back(k); ranges.push_back(1);
+    }
+    std::vector<float> im(4 * 13, 1.0f), com(4 * 13, 0.0f);
+    std::vector<float4> q;
+    std::vector<JointPhase> ph;
+    build_joint_program(t, ranges, im.data(), com.data(), q, ph);
+    auto u = [](float f) { uint32_t x; std::memcpy(&x, &f, 4); return x; };
+    for (size_t r = 0; r + kJRecQuads <= q.size(); r += kJRecQuads)
+        for (size_t h : {0, 4}) printf("%u %u %u %u\\n", u(q[r + h].x), u(q[r + h].y), u(q[r + h].z), u(q[r + h].w) >> 8);
+""")
+    assert rows == [[2 * k + 1, 2 * k + 2, k, t] for k, t in enumerate([2, 7, 3, 4, 5, 10]) for _ in range(2)]

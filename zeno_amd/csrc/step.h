@@ -253,9 +253,10 @@ constexpr uint32_t kJRecQuads = 8;  // float4 per solve record
 constexpr uint32_t kJHalfQuads = 4;  // float4 per lane-pair half record
 struct JointPhase { uint32_t type, start, count, com; };  // com: a body's centre of mass is off its origin
 
-// Record layout (float4 quads). q0 = (ia, ib, template index, flags) [u32], whose x and z the
-// kernel turns into byte offsets in the lane-pair types' halves; flags: bit0
-// inv_m_a > 0, bit1 inv_m_b > 0, bits 8-15 the constraint type.
+// Record layout (float4 quads). q0 = q4 = (ia, ib, template index, flags) [u32], the header of each
+// half, whose x and z the kernel turns into the byte offsets of the half's body and of the
+// multiplier; flags: bit0 inv_m_a > 0, bit1 inv_m_b > 0, bits 8-15 the constraint type. Every type
+// has both headers, as the lanes form their addresses before the type is told apart.
 // Lane-pair types (POSITIONAL, ANGULAR, ANGULAR_LIMIT) hold two halves, quads 0-3 for the
 // lane of body a and quads 4-7 for the lane of body b, each laid out as
 //   h0 = q0,  h1 = inverse mass and inertia of the lane's body,
@@ -263,11 +264,11 @@ struct JointPhase { uint32_t type, start, count, com; };  // com: a body's centr
 //        ANGULAR_LIMIT the limit axis; .w is replaced by compliance / dt^2 at kernel start,
 //   h3 = POSITIONAL the lane's centre of mass, ANGULAR_LIMIT (lower, upper), else 0,
 // so each lane reads only its own half and needs no selects between the two bodies.
-// Single-lane types (run by body a's lane) use quads 0-6:
+// Single-lane types (run by body a's lane):
 //   q1 / q2 = inverse mass and inertia of body a / b, q3.w = compliance (-> / dt^2),
-//   WELD:       q3.xyz anchor_a, q4.xyz anchor_b, q5 target quaternion
-//   LIN. LIMIT: q3.xyz axis, q4.xyz anchor_b, q5.xy (lower, upper)
-//   SLIDER:     q3.xyz anchor_a, q4.xyz anchor_b, q5.xyz axis, q6 target quaternion
+//   WELD:       q3.xyz anchor_a, q7.xyz anchor_b, q5 target quaternion
+//   LIN. LIMIT: q3.xyz axis, q7.xyz anchor_b, q5.xy (lower, upper)
+//   SLIDER:     q3.xyz anchor_a, q7.xyz anchor_b, q5.xyz axis, q6 target quaternion
 inline bool joint_type_solved(uint32_t t) {
     return t == C_POSITIONAL || t == C_ANGULAR || t == C_ANGULAR_LIMIT || t == C_LINEAR_LIMIT || t == C_WELD ||
            t == C_SLIDER;
@@ -334,19 +335,19 @@ inline void build_joint_program(const std::vector<ConstraintRec>& tmpl, const st
                             break;
                     }
                 } else {
-                    q[0] = head; q[1] = mia; q[2] = mib;
+                    q[0] = q[4] = head; q[1] = mia; q[2] = mib;
                     q[3] = make_float4(A[0], A[1], A[2], comp);
                     switch (type) {
                         case C_WELD:
-                            q[4] = make_float4(Bv[0], Bv[1], Bv[2], 0);
+                            q[7] = make_float4(Bv[0], Bv[1], Bv[2], 0);
                             q[5] = make_float4(t.axis_target[0], t.axis_target[1], t.axis_target[2], t.axis_target[3]);
                             break;
                         case C_LINEAR_LIMIT:
-                            q[4] = make_float4(Bv[0], Bv[1], Bv[2], 0);
+                            q[7] = make_float4(Bv[0], Bv[1], Bv[2], 0);
                             q[5] = make_float4(t.limits[0], t.limits[1], 0, 0);
                             break;
                         case C_SLIDER:
-                            q[4] = make_float4(Bv[0], Bv[1], Bv[2], 0);
+                            q[7] = make_float4(Bv[0], Bv[1], Bv[2], 0);
                             q[5] = make_float4(t.axis_target[0], t.axis_target[1], t.axis_target[2], 0);
                             q[6] = make_float4(t.limits[0], t.limits[1], t.limits[2], t.limits[3]);
                             break;

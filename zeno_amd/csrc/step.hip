@@ -236,16 +236,28 @@ __device__ __forceinline__ q4 qdelta_signed(f3 d, q4 q, float sg) { return qscal
 // and its centre of mass or the angular limits.
 struct JHalf { float4 h0, mi, v1, v2; };
 __device__ __forceinline__ JHalf load_half(const float4* p) { return JHalf{p[0], p[1], p[2], p[3]}; }
-// The header's x is the byte offset of the lane's body in the body arrays and its z the
-// multiplier's (fill_alpha, in the lane-pair types' records alone).
+// The state a lane-pair solve reads for the lane's body: position, orientation and the
+// constraint's multiplier.
+struct JState { float4 P, Q; float lam; };
+// In both halves of every record, of the single-lane types too, the header's x is the byte offset
+// of the half's body in the body arrays and its z the multiplier's (fill_alpha).
 template <int BS>
-__device__ __forceinline__ float4* jbody(const BodyArr<BS>& arr, const JHalf& h) {
-    return (float4*)((unsigned char*)arr.p + fbits(h.h0.x));
+__device__ __forceinline__ float4* jbody(const BodyArr<BS>& arr, uint32_t offset) {
+    return (float4*)((unsigned char*)arr.p + offset);
 }
+template <int BS>
+__device__ __forceinline__ float4* jbody(const BodyArr<BS>& arr, const JHalf& h) { return jbody(arr, fbits(h.h0.x)); }
 template <int BS>
 __device__ __forceinline__ float* jlam(const LdsT<BS>& s, const JHalf& h) {
     return (float*)((unsigned char*)s.lam + fbits(h.h0.z));
 }
+// Loaded before the type is told apart, so the compiler may place the reads; a type that does not use
+// them drops them.
+template <int BS>
+__device__ __forceinline__ JState load_jstate(const JHalf& h, const LdsT<BS>& s) {
+    return JState{*jbody(s.pos, h), *jbody(s.quat, h), *jlam(s, h)};
+}
+
 // Late selects. The positional and hinge solves evaluate their update unconditionally and
 // apply the reference's conditions (C > 1e-6, w > 1e-8, inverse mass > 0) only to the values
 // they store: a compare that feeds a branch or a select right away waits about 30 cycles for
@@ -262,14 +274,14 @@ __device__ __forceinline__ float* jlam(const LdsT<BS>& s, const JHalf& h) {
 // and a normalised quaternion has components within [-1, 1] or is the identity. Phases without
 // such a body, most of every robot's, skip the rotation (33 of about 300 instructions).
 template <int BS>
-__device__ __forceinline__ void solve_positional2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd, bool com) {
+__device__ __forceinline__ void solve_positional2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd, bool com) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
     const float sg = odd ? -1.0f : 1.0f;
-    const f3 P = xyz(*jbody(s.pos, h));
-    const q4 Q = toq(quat);
-    const float lambda_prev = *jlam(s, h);
+    const f3 P = xyz(st.P);
+    const q4 Q = toq(st.Q);
+    const float lambda_prev = st.lam;
     const f3 rr = qrot_fixed(xyz(h.v1), Q);                // r_a or r_b
     const f3 u = add(P, rr);                               // pos + r
     const f3 diff = sub(pair_a(u), pair_b(u));             // (pos_a + r_a) - (pos_b + r_b)
@@ -292,11 +304,11 @@ __device__ __forceinline__ void solve_positional2(const JHalf& h, float4 quat, c
 
 // :1131-1186 hinge axis alignment, lane pair.
 template <int BS>
-__device__ __forceinline__ void solve_angular2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd) {
+__device__ __forceinline__ void solve_angular2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
-    const q4 Q = toq(quat);
+    const q4 Q = toq(st.Q);
     const f3 axw = qrot_fixed(xyz(h.v1), Q);
     const f3 cr = cross(pair_a(axw), pair_b(axw));
     const float sin_angle = len_gate(cr);
@@ -313,14 +325,14 @@ __device__ __forceinline__ void solve_angular2(const JHalf& h, float4 quat, cons
 
 // :1189-1238 angular limit, lane pair.
 template <int BS>
-__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, float4 quat, const LdsT<BS>& s, bool odd) {
+__device__ __forceinline__ void solve_angular_limit2(const JHalf& h, const JState& st, const LdsT<BS>& s, bool odd) {
     const float alpha_tilde = h.v1.w;
     const float inv_mass = h.mi.x;
     const f3 iI = mk3(h.mi.y, h.mi.z, h.mi.w);
     const float sg = odd ? -1.0f : 1.0f;
     const f3 axis_local = xyz(h.v1);
     const float lower = h.v2.x, upper = h.v2.y;
-    const q4 Q = toq(quat);
+    const q4 Q = toq(st.Q);
     const q4 qa = pair_a(Q), qb = pair_b(Q);
     const q4 q_rel = qmul(qconj(qa), qb);
     const float angle = 2.0f * z_atan2f(dot(xyz(q_rel), axis_local), q_rel.w);
@@ -343,13 +355,13 @@ __device__ __forceinline__ void solve_angular_limit2(const JHalf& h, float4 quat
 // :1039-1129 weld (corrects body b only), one lane.
 template <int BS>
 __device__ __forceinline__ void solve_weld(const float4* r, const LdsT<BS>& s) {
-    const float4 q0 = r[0], mb = r[2], a3 = r[3], b4 = r[4], tg = r[5];
-    const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
+    const float4 mb = r[2], a3 = r[3], b4 = r[7], tg = r[5];
+    const uint32_t oa = fbits(r[0].x), ob = fbits(r[4].x);
     const float inv_mass_b = mb.x;
     const f3 iI_b = mk3(mb.y, mb.z, mb.w);
     const float alpha_tilde = a3.w;
-    const f3 pos_a = xyz(s.pos[ia]), pos_b = xyz(s.pos[ib]);
-    const q4 quat_a = toq(s.quat[ia]), quat_b = toq(s.quat[ib]);
+    const f3 pos_a = xyz(*jbody(s.pos, oa)), pos_b = xyz(*jbody(s.pos, ob));
+    const q4 quat_a = toq(*jbody(s.quat, oa)), quat_b = toq(*jbody(s.quat, ob));
     f3 r_a = qrot(xyz(a3), quat_a);
     f3 r_b = qrot(xyz(b4), quat_b);
     f3 diff = sub(add(pos_a, r_a), add(pos_b, r_b));
@@ -362,9 +374,9 @@ __device__ __forceinline__ void solve_weld(const float4* r, const LdsT<BS>& s) {
         if (w_b > 1e-8f) {
             float d_lambda = (-C) / (w_b + alpha_tilde);
             f3 impulse = sscale(d_lambda, n);
-            set_xyz(&s.pos[ib], sub(pos_b, scale(impulse, inv_mass_b)));
+            set_xyz(jbody(s.pos, ob), sub(pos_b, scale(impulse, inv_mass_b)));
             qb = qnormalize(qsub(quat_b, qdelta(mul(cross(r_b, impulse), iI_b), quat_b)));
-            s.quat[ib] = tof4(qb);
+            *jbody(s.quat, ob) = tof4(qb);
         }
     }
     const q4 target = toq(tg);
@@ -381,7 +393,7 @@ __device__ __forceinline__ void solve_weld(const float4* r, const LdsT<BS>& s) {
         if (w_b > 1e-8f) {
             float d_lambda_ang = angle / (w_b + alpha_tilde);
             f3 ang_impulse = sscale(d_lambda_ang, aw);
-            if (inv_mass_b > 0) s.quat[ib] = tof4(qnormalize(qsub(qb, qdelta(mul(ang_impulse, iI_b), qb))));
+            if (inv_mass_b > 0) *jbody(s.quat, ob) = tof4(qnormalize(qsub(qb, qdelta(mul(ang_impulse, iI_b), qb))));
         }
     }
 }
@@ -389,15 +401,15 @@ __device__ __forceinline__ void solve_weld(const float4* r, const LdsT<BS>& s) {
 // :1241-1293 linear limit, one lane.
 template <int BS>
 __device__ __forceinline__ void solve_linear_limit(const float4* r, const LdsT<BS>& s) {
-    const float4 q0 = r[0], ma = r[1], mb = r[2], a3 = r[3], b4 = r[4], lim = r[5];
-    const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
+    const float4 ma = r[1], mb = r[2], a3 = r[3], b4 = r[7], lim = r[5];
+    const uint32_t oa = fbits(r[0].x), ob = fbits(r[4].x);
     const float inv_mass_a = ma.x, inv_mass_b = mb.x;
     const f3 iI_a = mk3(ma.y, ma.z, ma.w), iI_b = mk3(mb.y, mb.z, mb.w);
     const float alpha_tilde = a3.w;
     const f3 axis_local = xyz(a3);
     const float lower = lim.x, upper = lim.y;
-    const f3 pos_a = xyz(s.pos[ia]), pos_b = xyz(s.pos[ib]);
-    const q4 qa = toq(s.quat[ia]), qb = toq(s.quat[ib]);
+    const f3 pos_a = xyz(*jbody(s.pos, oa)), pos_b = xyz(*jbody(s.pos, ob));
+    const q4 qa = toq(*jbody(s.quat, oa)), qb = toq(*jbody(s.quat, ob));
     f3 r_a = qrot(mk3(0.0f, 0.0f, 0.0f), qa);
     f3 r_b = qrot(xyz(b4), qb);
     f3 aw = qrot(axis_local, qa);
@@ -413,8 +425,8 @@ __device__ __forceinline__ void solve_linear_limit(const float4* r, const LdsT<B
         if (w > 1e-8f) {
             float d_lambda = abs_v / (w + alpha_tilde);
             f3 impulse = sscale(d_lambda, n);
-            if (inv_mass_a > 0) set_xyz(&s.pos[ia], sub(pos_a, scale(impulse, inv_mass_a)));
-            if (inv_mass_b > 0) set_xyz(&s.pos[ib], add(pos_b, scale(impulse, inv_mass_b)));
+            if (inv_mass_a > 0) set_xyz(jbody(s.pos, oa), sub(pos_a, scale(impulse, inv_mass_a)));
+            if (inv_mass_b > 0) set_xyz(jbody(s.pos, ob), add(pos_b, scale(impulse, inv_mass_b)));
         }
     }
 }
@@ -422,13 +434,13 @@ __device__ __forceinline__ void solve_linear_limit(const float4* r, const LdsT<B
 // :1296-1399 slider, one lane.
 template <int BS>
 __device__ __forceinline__ void solve_slider(const float4* r, const LdsT<BS>& s) {
-    const float4 q0 = r[0], ma = r[1], mb = r[2], a3 = r[3], b4 = r[4], ax = r[5], tg = r[6];
-    const uint32_t ia = fbits(q0.x), ib = fbits(q0.y);
+    const float4 ma = r[1], mb = r[2], a3 = r[3], b4 = r[7], ax = r[5], tg = r[6];
+    const uint32_t oa = fbits(r[0].x), ob = fbits(r[4].x);
     const float inv_mass_a = ma.x, inv_mass_b = mb.x;
     const f3 iI_a = mk3(ma.y, ma.z, ma.w), iI_b = mk3(mb.y, mb.z, mb.w);
     const float alpha_tilde = a3.w;
-    const f3 pos_a = xyz(s.pos[ia]), pos_b = xyz(s.pos[ib]);
-    const q4 quat_a = toq(s.quat[ia]), quat_b = toq(s.quat[ib]);
+    const f3 pos_a = xyz(*jbody(s.pos, oa)), pos_b = xyz(*jbody(s.pos, ob));
+    const q4 quat_a = toq(*jbody(s.quat, oa)), quat_b = toq(*jbody(s.quat, ob));
     f3 r_a = qrot(xyz(a3), quat_a);
     f3 r_b = qrot(xyz(b4), quat_b);
     f3 diff = sub(add(pos_a, r_a), add(pos_b, r_b));
@@ -444,11 +456,11 @@ __device__ __forceinline__ void solve_slider(const float4* r, const LdsT<BS>& s)
         float d_lambda = (-perp_len) / (w + alpha_tilde);
         f3 impulse = sscale(d_lambda, n);
         if (inv_mass_a > 0) {
-            set_xyz(&s.pos[ia], add(pos_a, scale(impulse, inv_mass_a)));
+            set_xyz(jbody(s.pos, oa), add(pos_a, scale(impulse, inv_mass_a)));
             qa = qnormalize(qadd(quat_a, qdelta(mul(cross(r_a, impulse), iI_a), quat_a)));
         }
         if (inv_mass_b > 0) {
-            set_xyz(&s.pos[ib], sub(pos_b, scale(impulse, inv_mass_b)));
+            set_xyz(jbody(s.pos, ob), sub(pos_b, scale(impulse, inv_mass_b)));
             qb = qnormalize(qsub(quat_b, qdelta(mul(cross(r_b, impulse), iI_b), quat_b)));
         }
     }
@@ -469,8 +481,8 @@ __device__ __forceinline__ void solve_slider(const float4* r, const LdsT<BS>& s)
             if (inv_mass_b > 0) qb = qnormalize(qsub(qb, qdelta(mul(ang_impulse, iI_b), qb)));
         }
     }
-    if (inv_mass_a > 0) s.quat[ia] = tof4(qa);
-    if (inv_mass_b > 0) s.quat[ib] = tof4(qb);
+    if (inv_mass_a > 0) *jbody(s.quat, oa) = tof4(qa);
+    if (inv_mass_b > 0) *jbody(s.quat, ob) = tof4(qb);
 }
 
 // Inclusive max-scan of v over segments of G lanes (sl = lane within the segment): DPP row
@@ -768,21 +780,16 @@ __device__ __forceinline__ void narrow_slot(const StepArgs& a, const Mdl& md, co
     }
 }
 
-// One joint solve of the given type on the lane pair: h is the lane's half record (lane-pair
-// types), r the whole record in LDS (single-lane types, run by body a's lane). The body's state is
-// read for the lane-pair types alone: of a single-lane record only the first half starts with a
-// header, and its fields are indices, not byte offsets. The orientation is read before the types
-// are told apart, the position and the multiplier by the one type that uses them.
+// One joint solve of the given type on the lane pair: h is the lane's half record and st its
+// body's state (lane-pair types), r the whole record in LDS (single-lane types, run by body
+// a's lane, which read the state themselves).
 template <int BS>
-__device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const float4* r, const LdsT<BS>& s, bool odd) {
-    if (joint_type_paired(type)) {
-        const float4 quat = *jbody(s.quat, h);
-        if (type == C_POSITIONAL) solve_positional2(h, quat, s, odd, com);
-        else if (type == C_ANGULAR) solve_angular2(h, quat, s, odd);
-        else solve_angular_limit2(h, quat, s, odd);
-        return;
-    }
+__device__ __forceinline__ void solve_joint(uint32_t type, bool com, const JHalf& h, const JState& st, const float4* r,
+                                            const LdsT<BS>& s, bool odd) {
     switch (type) {
+        case C_POSITIONAL: solve_positional2(h, st, s, odd, com); break;
+        case C_ANGULAR: solve_angular2(h, st, s, odd); break;
+        case C_ANGULAR_LIMIT: solve_angular_limit2(h, st, s, odd); break;
         case C_WELD: if (!odd) solve_weld(r, s); break;
         case C_LINEAR_LIMIT: if (!odd) solve_linear_limit(r, s); break;
         case C_SLIDER: if (!odd) solve_slider(r, s); break;
@@ -1632,14 +1639,14 @@ void step_kernel(StepArgs a) {
             if (joint_type_paired((fbits(q[0].w) >> 8) & 0xFFu)) {
                 q[2].w = q[2].w / (a.dt * a.dt);
                 q[6].w = q[6].w / (a.dt * a.dt);
-                // Each half's header: its own body and the multiplier, as byte offsets.
-                q[0].x = __uint_as_float(fbits(q[0].x) * (16u * (uint32_t)BS));
-                q[4].x = __uint_as_float(fbits(q[4].y) * (16u * (uint32_t)BS));
-                q[0].z = __uint_as_float(fbits(q[0].z) * 4u);
-                q[4].z = __uint_as_float(fbits(q[4].z) * 4u);
             } else {
                 q[3].w = q[3].w / (a.dt * a.dt);
             }
+            // Each half's header: its own body and the multiplier, as byte offsets.
+            q[0].x = __uint_as_float(fbits(q[0].x) * (16u * (uint32_t)BS));
+            q[4].x = __uint_as_float(fbits(q[4].y) * (16u * (uint32_t)BS));
+            q[0].z = __uint_as_float(fbits(q[0].z) * 4u);
+            q[4].z = __uint_as_float(fbits(q[4].z) * 4u);
         }
     };
     if (PL == PL_LDS) {
@@ -2832,11 +2839,12 @@ void step_kernel(StepArgs a) {
                     const uint32_t st = __builtin_amdgcn_readfirstlane(ph1.start), cn = __builtin_amdgcn_readfirstlane(ph1.count);
                     nxt = load_half(md.jrec + (st + (kf < cn ? kf : 0u)) * kJRecQuads + half);
                 }
-                if (live && kf < cnt) solve_joint(type, com, cur, md.jrec + (start + kf) * kJRecQuads, s, odd);
+                if (live && kf < cnt) solve_joint(type, com, cur, load_jstate(cur, s), md.jrec + (start + kf) * kJRecQuads, s, odd);
                 if (live) {
                     for (uint32_t k = kf + G / 2; k < cnt; k += G / 2) {
                         const float4* r = md.jrec + (start + k) * kJRecQuads;
-                        solve_joint(type, com, load_half(r + half), r, s, odd);
+                        const JHalf hk = load_half(r + half);
+                        solve_joint(type, com, hk, load_jstate(hk, s), r, s, odd);
                     }
                 }
                 wave_sync<HBM>();
