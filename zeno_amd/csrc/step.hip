@@ -80,7 +80,9 @@ struct LdsT {
     uint32_t* gmeta;         // staged geom body | type << 16
     float* obs;              // the observation row (stage L), written back with the state
     uint2* stash;            // contact pool: (bodies, geoms) of each slot
-    unsigned long long *runs, *vmask, *wmask;  // contact pool: bits per slot (see list_pass, fill_pool)
+    // Contact pool, a bit per slot: a run of the snapshot starts here; the slot is in contact; the
+    // list's record does not say "no contact" yet.
+    unsigned long long *runs, *vmask, *wmask;
     uint32_t* misc;
 };
 
@@ -3067,9 +3069,34 @@ void step_kernel(StepArgs a) {
         if (do_prep) {
         ContactRec* gc = a.contacts + (size_t)env * M;
         if constexpr (POOL) {
-            if (hv.contacts) {
+            // The view was current before this launch. One substep that neither appends nor sorts
+            // (the list's count is written below) has changed the slots that are in contact now or
+            // were before, few of a robot's 64; otherwise the whole list is stored, 4 KB over PCIe for
+            // an environment, which takes far longer than the step (24000 walkers 1850 -> 165 us).
+            auto store_view = [&](const auto& k) {
+                if (!k.hv.contacts) return;
                 wave_sync<true>();
-                for (uint32_t k = sl; k < n_out; k += G) copy_record(&hv.contacts[(size_t)env * M + k], &list[k]);
+                const size_t first = (size_t)env * k.M;
+                const unsigned char* const set = smem + (PL == PL_LDS ? k.ml.bytes : 0u) + (grp * EPW + le) * k.lds.bytes;
+                const unsigned long long* const now = (const unsigned long long*)(set + k.lds.vmask);
+                const unsigned long long* const before = (const unsigned long long*)(set + k.lds.wmask);
+                const uint32_t had = k.counts[env];
+                const bool all = total != 1u || k.sort_all != 0u || had < k.M || had > 0xFFFFFFFFu - k.P;
+                for (uint32_t i = sl; i < n_out; i += G) {
+                    if (all || (((now[i >> 6] | before[i >> 6]) >> (i & 63u)) & 1ull) != 0ull)
+                        copy_record(&k.hv.contacts[first + i], &k.contacts[first + i]);
+                }
+            };
+            if constexpr (SPLIT) {
+                // The arguments are read anew: kept from the kernel's start they are scalar registers
+                // that the loops above spill around (269 spills against 307 at four environments a
+                // wave, and up to 1% of a robot's step).
+                using Args = const __attribute__((address_space(4))) StepArgs;
+                Args* k = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(k));
+                store_view(*k);
+            } else {
+                store_view(a);
             }
         } else
         for (uint32_t k = sl; k < n_out; k += G) {

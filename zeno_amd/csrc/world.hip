@@ -501,7 +501,9 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
     a.hv.jvel = (float*)view(MIR_JVEL);
     a.hv.jtrq = (float*)view(MIR_JTRQ);
     a.hv.obs = (float*)view(MIR_OBS);
-    a.hv.contacts = (ContactRec*)view(MIR_CON);
+    // The kernel stores the slots that it changes, so into a view that is current alone.
+    const bool list_behind = dirty[MIR_CON];
+    a.hv.contacts = list_behind ? nullptr : (ContactRec*)view(MIR_CON);
     a.hv.counts = (uint32_t*)view(MIR_COUNT);
     hipEvent_t t0 = nullptr, t1 = nullptr;
     // Under capture the launch becomes a graph node; event timing and profiling stay eager-only.
@@ -527,12 +529,13 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
     ZA_TRY(launch_step(a, epw, waves, stream, split));
     if (prof_events) { ZA_TRY(hipEventRecord(prof_stop, stream)); prof_pending = true; }
     if (timed) ZA_TRY(hipEventRecord(t1, stream));
+    if (capturing) return hipSuccess;  // nothing has run
     mark_all_dirty();
     // The held views were current before this launch (every state-changing call leaves them
     // so) and the kernel stores what it changes in them: they are current once the stream
     // reaches this point.
     for (int i = 0; i < MIR_COUNT_ALL; ++i) {
-        if (direct && exposed[i]) { dirty[i] = false; views_pending = true; }
+        if (exposed[i] && !(i == MIR_CON && list_behind)) { dirty[i] = false; views_pending = true; }
     }
     return hipSuccess;
 }
