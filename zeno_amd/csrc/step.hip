@@ -1,12 +1,20 @@
 // Fused physics step for CDNA4 (gfx950).
 //
-// One wave steps EPW environments; each environment owns G = 64 / EPW lanes and an LDS
-// working set (bodies, joint state, lambdas, the contact list and the previous-contact
-// snapshot). A workgroup holds up to four such groups sharing one LDS copy of the model
-// records, and in the split shapes each group has a second wave that runs the contact
-// pipeline while the first solves the joints (see step_kernel). A launch runs every substep
-// of one zeno_world_step call, so HBM is read once and written once per call while all
+// One wave steps EPW environments; each environment owns G = 64 / EPW lanes and a working set
+// (bodies, joint state, lambdas, contact data). A workgroup holds up to four such groups sharing
+// one LDS copy of the model records, and in the split shapes each group has a second wave that
+// runs the contact pipeline while the first solves the joints (see step_kernel). A launch runs
+// every substep of one zeno_world_step call, or of several consecutive ones of a captured
+// schedule, so the bodies' state is read from HBM once and written once per launch while all
 // solver iterations stay in LDS.
+//
+// Where the contact list lives. Without the spatial hash and with the working sets in LDS, the
+// list stays in the state's array in HBM: each substep reads its slots' bodies and geoms, keeps the
+// slots that the narrow phase finds in contact in a pool in LDS (make_env_pool), and writes those
+// back, with "no contact" for the ones that were in contact before. A list that a substep appends
+// to or sorts is copied to a scratch list first, as the previous contacts to match; a full list is
+// its own copy. With the hash, or with the working sets in HBM, the list, the previous contacts and
+// a logical->physical permutation of its slots are part of the working set.
 //
 // Stage order and arithmetic follow World.stepOnce (src/world/world.zig:934-1293) and the
 // MSL kernels of src/shaders/all_shaders.metal, cited per stage. Where the reference runs
@@ -16,9 +24,10 @@
 //   S3 joint constraints per colour (bodies in one colour are disjoint);
 //   S4 contact slots Gauss-Seidel in slot order: slots are levelled so that a slot runs
 //      after every earlier slot sharing a body it writes, then levels run in order.
-// The stable contact sort (all_shaders.metal:711-745) is a rank sort over a logical->physical
-// permutation, so 64-byte records never move in LDS; the permutation is applied when the
-// list is written back.
+// The stable contact sort (all_shaders.metal:711-745) is a rank sort, or a bitonic one of (key,
+// slot) for long lists, and runs only where a substep appended: in HBM the records that change
+// places move through a scratch list, in a working set the permutation alone is sorted and the
+// 64-byte records move when the list is written back.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -487,21 +496,11 @@ __device__ __forceinline__ void solve_slider(const float4* r, const LdsT<BS>& s)
     if (inv_mass_b > 0) *jbody(s.quat, ob) = tof4(qb);
 }
 
-// Inclusive max-scan of v over segments of G lanes (sl = lane within the segment): DPP row
-// shifts when a segment lies inside one 16-lane row, LDS-backed shuffles otherwise.
-template <int G>
-__device__ __forceinline__ uint32_t seg_max_scan(uint32_t v, uint32_t sl) {
-    if constexpr (G <= 16) {
-        auto step = [&](uint32_t t, uint32_t d) { if (sl >= d) v = t > v ? t : v; };
-        if constexpr (G > 1) step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false), 1);  // row_shr:1
-        if constexpr (G > 2) step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false), 2);  // row_shr:2
-        if constexpr (G > 4) step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false), 4);  // row_shr:4
-        if constexpr (G > 8) step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false), 8);  // row_shr:8
-    } else {
-        for (uint32_t d = 1; d < (uint32_t)G; d <<= 1) {
-            const uint32_t t = __shfl_up(v, d, G);
-            if (sl >= d) v = t > v ? t : v;
-        }
+// Inclusive max-scan of v over the wave.
+__device__ __forceinline__ uint32_t wave_max_scan(uint32_t v, uint32_t lane) {
+    for (uint32_t d = 1; d < (uint32_t)kWave; d <<= 1) {
+        const uint32_t t = __shfl_up(v, d);
+        if (lane >= d) v = t > v ? t : v;
     }
     return v;
 }
@@ -1439,10 +1438,10 @@ __device__ __forceinline__ uint32_t spill_levels(const SpillArrays& sp, const F&
 // there each wave steps its own environments and synchronises with itself only.
 // SPLIT: two waves per group of EPW environments, on the same SIMD (wave w and wave w + NG of
 // a workgroup of 2 NG waves). The solver wave runs stages A-D, the joint and contact solves
-// and the post-solve stages; the helper wave runs the snapshot, the broad phase, the sort, the
-// narrow phase, the cache matching and the contact levels while the solver runs the joints
-// (these read the poses after integration and write nothing the joint solve reads), and
-// writes the contact list back while the solver finishes. The solver leaves the poses after
+// and the post-solve stages; the helper wave reads the list while the solver integrates, runs the
+// broad phase, the sort, the narrow phase, the cache matching and the contact levels while the
+// solver runs the joints (these read the poses after integration and write nothing the joint
+// solve reads), and writes the slots in contact back to the list while the solver finishes. The solver leaves the poses after
 // integration in the force and torque arrays (dead until the next substep) for the helper, as
 // the joint solve moves the bodies meanwhile. Three workgroup barriers per substep order the
 // two: after integration, before the contact solve and after it.
@@ -1463,6 +1462,7 @@ void step_kernel(StepArgs a) {
     static_assert(!HASH || EPW == 1, "the spatial hash runs one environment per workgroup");
     static_assert(!GROUP || EPW == 1, "type-grouped narrow phase: one environment per workgroup");
     static_assert(!SPLIT || (PL == PL_LDS && !HASH && !GROUP), "split groups: working sets and model in LDS");
+    static_assert(POOL || G == kWave, "a list in the working set belongs to a whole wave");
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = (int)(threadIdx.x & (kWave - 1));    // lane
     constexpr bool MULTI = PL == PL_LDS && !HASH;          // several waves per workgroup possible
@@ -1572,10 +1572,8 @@ void step_kernel(StepArgs a) {
         if (j0 < Jp) p_jt = a.jtrq[(size_t)env * Jp + j0];
         if (j0 < N) p_lam = a.lam[(size_t)env * N + j0];
     }
-    // The contact list and counts, read ahead into registers (one wave per group). A split
-    // group's helper reads them after the first barrier of the first substep instead, straight
-    // into LDS: the contact records are most of the bytes, and the helper needs them only after
-    // integration, while the solver's body reads then meet no contact traffic.
+    // The counts, and of a list in the working set the slots, read ahead into registers. (A split
+    // group's helper reads the counts once the model records are in LDS.)
     auto load_contacts = [&]() {
         if constexpr (POOL) {
             count = a.counts[env];
@@ -1750,9 +1748,7 @@ void step_kernel(StepArgs a) {
             s = bind_lds<BS>(env_base + at, a.lds);
         }
         // ---- Previous-contact snapshot (cache_contacts of the last substep) -----------
-        // A split group's helper takes it after the first barrier of the substep (with the
-        // contact list's LDS copy in the first substep), so the solver never waits for it.
-        // Taken after the broad phase (LATE_SNAP), its slots at or past the count the broad
+        // With the list in the working set (the contact pool's is below). Taken after the broad phase (LATE_SNAP), its slots at or past the count the broad
         // phase started from (`kept`) may hold appends: a list whose count the host lowered or
         // reset before this call. The first substep reads those from the call's list in HBM,
         // as loaded (the permutation is still the identity); in later substeps the snapshot's
@@ -2325,15 +2321,8 @@ void step_kernel(StepArgs a) {
                     }
                 }
             } else {
-                // One environment per wave here (the long lists need EPW 1 or 2 to fit LDS);
-                // the network runs to the wave's largest padded length.
                 uint32_t np = 1;
                 while (np < n) np <<= 1;
-                uint32_t wave_np = need ? np : 1u;
-                for (uint32_t d = 1; d < 64u; d <<= 1) {
-                    const uint32_t t = __shfl_xor(wave_np, d);
-                    wave_np = t > wave_np ? t : wave_np;
-                }
                 if (need) {
                     for (uint32_t k = sl; k < np; k += G) {
                         uint32_t key = 0xFFFFFFFFu;
@@ -2346,9 +2335,9 @@ void step_kernel(StepArgs a) {
                     }
                 }
                 wave_sync<HBM>();
-                for (uint32_t kk = 2; kk <= wave_np; kk <<= 1) {
+                for (uint32_t kk = 2; kk <= np; kk <<= 1) {
                     for (uint32_t j = kk >> 1; j > 0; j >>= 1) {
-                        if (need && kk <= np) {
+                        if (need) {
                             for (uint32_t t = sl; t < np / 2; t += G) {
                                 const uint32_t i = ((t & ~(j - 1u)) << 1) | (t & (j - 1u));
                                 const uint32_t l = i | j;
@@ -2534,28 +2523,19 @@ void step_kernel(StepArgs a) {
                 const uint32_t* idx = s.con[phys].indices;
                 return (geom_type(idx[2]) & 7u) * 8u + (geom_type(idx[3]) & 7u);
             };
-            constexpr uint32_t kPer = 64u / G;  // classes per lane
-            for (uint32_t i = 0; i < kPer; ++i) ccount[sl * kPer + i] = 0u;
+            ccount[sl] = 0u;  // a class per lane
             wave_sync<HBM>();
             if (live) {
                 for (uint32_t k = sl; k < n_live; k += G) atomicAdd(&ccount[slot_class(s.perm[k])], 1u);
             }
             wave_sync<HBM>();
-            // Exclusive scan of the env's 64 counters: each lane sums its kPer classes, the
-            // env's G lanes scan those sums, and each lane writes its classes' offsets.
-            uint32_t sum = 0;
-            for (uint32_t i = 0; i < kPer; ++i) sum += ccount[sl * kPer + i];
+            const uint32_t sum = ccount[sl];
             uint32_t incl = sum;
             for (int d = 1; d < G; d <<= 1) {
                 const uint32_t t = __shfl_up(incl, d, G);
                 if (sl >= d) incl += t;
             }
-            uint32_t run = incl - sum;
-            for (uint32_t i = 0; i < kPer; ++i) {
-                const uint32_t c = ccount[sl * kPer + i];
-                ccount[sl * kPer + i] = run;
-                run += c;
-            }
+            ccount[sl] = incl - sum;
             wave_sync<HBM>();
             if (live) {
                 for (uint32_t k = sl; k < n_live; k += G) {
@@ -2589,10 +2569,10 @@ void step_kernel(StepArgs a) {
                 const uint32_t i = base + sl;
                 uint32_t v = 0;
                 if (i < pn && i > 0 && key_at(i - 1) != key_at(i)) v = i;
-                v = seg_max_scan<G>(v, sl);
+                v = wave_max_scan(v, (uint32_t)sl);
                 v = carry > v ? carry : v;
                 if (i < pn) rstart[i] = v;
-                carry = __shfl(v, G - 1, G);
+                carry = __shfl(v, kWave - 1);
             }
         }
         wave_sync<HBM>();
