@@ -515,7 +515,7 @@ struct StepArgs {
     const ContactRec* prev_contacts; // [E*M]
     // Contact pool: two scratch lists per environment (the snapshot of a list that this substep
     // changes, or the levels of a pool too long for LDS; sorted records, or that pool), and the
-    // working list of environments that a step mask holds back.
+    // working list of environments that a step mask holds back; of this launch's environments.
     ContactRec* list_snap;          // [E*M]
     ContactRec* list_tmp;           // [E*M]
     ContactRec* list_masked;        // [E*M]

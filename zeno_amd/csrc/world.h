@@ -65,9 +65,12 @@ struct World {
     float *d_jpos = nullptr, *d_jvel = nullptr, *d_jtrq = nullptr, *d_obs = nullptr, *d_lam = nullptr;
     float* d_actions = nullptr;
     ContactRec* d_con = nullptr;
-    // Contact pool (working sets in LDS without the spatial hash): scratch lists of every
-    // environment, and the working lists of environments a step mask holds back (on first use).
+    // Contact pool (working sets in LDS without the spatial hash): two scratch lists of M records
+    // for each of `list_envs` environments, and the working lists of those that a step mask holds
+    // back (on first use). list_envs is E unless device memory did not hold that much: a launch then
+    // runs in parts of list_envs environments, one after another on the stream.
     ContactRec *d_list_snap = nullptr, *d_list_tmp = nullptr, *d_list_masked = nullptr;
+    uint32_t list_envs = 0;
     uint32_t *d_counts = nullptr, *d_pcounts = nullptr;
     uint32_t* d_cell_ids = nullptr;       // [E*G] hash mode
     // Count-only sweep of a full list: the non-plane geoms (at most 64; none when the scene
@@ -163,6 +166,10 @@ struct World {
     hipError_t stage_actions(const float* actions, const float** d_out);
     hipError_t mark_actions_used();
     hipError_t upload_mask(const uint8_t* mask, uint8_t** d_out);
+    hipError_t alloc_lists(uint32_t envs);
+    void free_lists();
+    // Device memory for `count` elements; where there is too little, from the scratch lists' share.
+    template <typename T> hipError_t grow(T** p, size_t count);
     hipError_t ensure_subset_buffers();
     hipError_t write_state_array(float4* dst, MirrorId mid, const float* src, const uint8_t* mask);
     const void* device_src(MirrorId id) const;

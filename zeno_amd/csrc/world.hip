@@ -67,6 +67,27 @@ __global__ void fill_u8_kernel(uint8_t* p, uint32_t n, uint8_t v) {
     if (i < n) p[i] = v;
 }
 
+// The arguments of a launch over `count` environments from `first` on: every per-environment array
+// moved along, but for the scratch lists.
+StepArgs step_part(const StepArgs& a, uint32_t first, uint32_t count) {
+    StepArgs p = a;
+    p.E = count;
+    auto move = [&](auto*& ptr, size_t stride) { if (ptr) ptr += (size_t)first * stride; };
+    for (float4** q : {&p.pos, &p.quat, &p.vel, &p.angvel, &p.acc, &p.hv.pos, &p.hv.quat, &p.hv.vel, &p.hv.angvel, &p.hv.acc}) move(*q, a.B);
+    for (float** q : {&p.jpos, &p.jvel, &p.jtrq, &p.hv.jpos, &p.hv.jvel, &p.hv.jtrq}) move(*q, a.Jp);
+    for (float** q : {&p.obs, &p.hv.obs}) move(*q, a.obsp);
+    for (uint32_t** q : {&p.counts, &p.pcounts, &p.hv.counts}) move(*q, 1);
+    move(p.lam, a.N);
+    move(p.actions, a.A);
+    for (ContactRec** q : {&p.contacts, &p.prev_out, &p.hv.contacts}) move(*q, a.M);
+    move(p.prev_contacts, a.M);
+    move(p.prev_detached, 1);
+    move(p.prev_detached_out, 1);
+    move(p.step_mask, 1);
+    if (first > 0) p.phase_ticks = nullptr;  // the first workgroup's
+    return p;
+}
+
 inline uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
 template <typename T>
@@ -392,11 +413,13 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     if ((e = dalloc(w, &w->d_counts, w->E)) != hipSuccess) return fail("hipMalloc", e);
     if ((e = dalloc(w, &w->d_pcounts, w->E)) != hipSuccess) return fail("hipMalloc", e);
     if (w->hash && (e = dalloc(w, &w->d_cell_ids, (size_t)w->E * m.num_geoms)) != hipSuccess) return fail("hipMalloc", e);
-    if (!w->hash && w->placement <= PL_MODEL_HBM) {
-        if ((e = dalloc(w, &w->d_list_snap, (size_t)w->E * std::max<uint32_t>(w->M, 1))) != hipSuccess) return fail("hipMalloc", e);
-        if ((e = dalloc(w, &w->d_list_tmp, (size_t)w->E * std::max<uint32_t>(w->M, 1))) != hipSuccess) return fail("hipMalloc", e);
-    }
     if (w->placement >= PL_ALL_HBM && (e = dalloc(w, &w->d_work, (size_t)w->E * w->lds.bytes)) != hipSuccess) return fail("hipMalloc", e);
+    if (!w->hash && w->placement <= PL_MODEL_HBM) {
+        // ZENO_AMD_LIST_ENVS=n (tests of launches in parts) starts from n environments' lists.
+        const char* env = std::getenv("ZENO_AMD_LIST_ENVS");
+        const int n = env ? std::atoi(env) : 0;
+        if ((e = w->alloc_lists(n > 0 ? std::min((uint32_t)n, w->E) : w->E)) != hipSuccess) return fail("hipMalloc", e);
+    }
     struct Z { void* p; size_t n; } zeros[] = {
         {w->d_pos, EB * 16}, {w->d_quat, EB * 16}, {w->d_vel, EB * 16}, {w->d_angvel, EB * 16}, {w->d_acc, EB * 16},
         {w->d_jpos, (size_t)w->E * w->Jp * 4}, {w->d_jvel, (size_t)w->E * w->Jp * 4}, {w->d_jtrq, (size_t)w->E * w->Jp * 4},
@@ -440,6 +463,47 @@ World* World::create(const Scene& scene, const ZenoConfig& cfg, std::string& err
     if ((e = hipHostMalloc((void**)&w->h_mask_stage, w->E, hipHostMallocDefault)) != hipSuccess) return fail("hipHostMalloc", e);
     if ((e = hipStreamSynchronize(w->stream)) != hipSuccess) return fail("init", e);
     return w;
+}
+
+// The lists of `envs` environments, or of half as many until device memory holds them; not fewer
+// than kMinListEnvs (a launch of fewer leaves most of the GPU idle).
+constexpr uint32_t kMinListEnvs = 1024;
+hipError_t World::alloc_lists(uint32_t envs) {
+    const bool masked = d_list_masked != nullptr;
+    free_lists();
+    for (;; envs = (envs + 1) / 2) {
+        list_envs = envs;
+        const size_t n = (size_t)envs * std::max<uint32_t>(M, 1);
+        hipError_t e = dalloc(this, &d_list_snap, n);
+        if (e == hipSuccess) e = dalloc(this, &d_list_tmp, n);
+        if (e == hipSuccess && masked) e = dalloc(this, &d_list_masked, n);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        free_lists();
+        if (e != hipErrorOutOfMemory || envs <= kMinListEnvs) return e;
+    }
+}
+
+void World::free_lists() {
+    for (ContactRec** p : {&d_list_snap, &d_list_tmp, &d_list_masked}) {
+        if (!*p) continue;
+        hipFree(*p);
+        *p = nullptr;
+        device_bytes -= (size_t)list_envs * std::max<uint32_t>(M, 1) * sizeof(ContactRec);
+    }
+}
+
+template <typename T>
+hipError_t World::grow(T** p, size_t count) {
+    hipError_t e = dalloc(this, p, count);
+    while (e == hipErrorOutOfMemory && d_list_snap && list_envs > kMinListEnvs) {
+        (void)hipGetLastError();
+        release_graph();  // captured launches hold the lists' addresses
+        ZA_TRY(hipStreamSynchronize(stream));
+        ZA_TRY(alloc_lists((list_envs + 1) / 2));
+        e = dalloc(this, p, count);
+    }
+    return e;
 }
 
 void World::mark_all_dirty() {
@@ -526,7 +590,12 @@ hipError_t World::launch(const float* d_act, uint32_t substeps, const uint8_t* d
         if (!prof_start) { ZA_TRY(hipEventCreate(&prof_start)); ZA_TRY(hipEventCreate(&prof_stop)); }
         ZA_TRY(hipEventRecord(prof_start, stream));
     }
-    ZA_TRY(launch_step(a, epw, waves, stream, split));
+    if (!d_list_snap || list_envs >= E) {
+        ZA_TRY(launch_step(a, epw, waves, stream, split));
+    } else {
+        for (uint32_t first = 0; first < E; first += list_envs)
+            ZA_TRY(launch_step(step_part(a, first, std::min(list_envs, E - first)), epw, waves, stream, split));
+    }
     if (prof_events) { ZA_TRY(hipEventRecord(prof_stop, stream)); prof_pending = true; }
     if (timed) ZA_TRY(hipEventRecord(t1, stream));
     if (capturing) return hipSuccess;  // nothing has run
@@ -718,20 +787,29 @@ hipError_t World::graph_launch() {
 }
 
 hipError_t World::ensure_subset_buffers() {
-    if (d_list_snap && !d_list_masked) ZA_TRY(dalloc(this, &d_list_masked, (size_t)E * std::max<uint32_t>(M, 1)));
     if (!d_prev_con) {
         release_graph();  // captured launches hold the buffer addresses of capture time
-        ZA_TRY(dalloc(this, &d_prev_con, (size_t)E * std::max<uint32_t>(M, 1)));
-        ZA_TRY(dalloc(this, &d_prev_detached, E));
+        ZA_TRY(grow(&d_prev_con, (size_t)E * std::max<uint32_t>(M, 1)));
+    }
+    if (!d_prev_detached) {
+        ZA_TRY(grow(&d_prev_detached, E));
         hipLaunchKernelGGL(fill_u8_kernel, dim3(blocks_for(E, 256)), dim3(256), 0, stream, d_prev_detached, E, (uint8_t)0);
         ZA_TRY(hipGetLastError());
+    }
+    while (d_list_snap && !d_list_masked) {
+        const uint32_t envs = list_envs;
+        ContactRec* list = nullptr;
+        ZA_TRY(grow(&list, (size_t)envs * std::max<uint32_t>(M, 1)));
+        if (envs == list_envs) { d_list_masked = list; break; }
+        hipFree(list);  // the other lists were made shorter for it
+        device_bytes -= (size_t)envs * std::max<uint32_t>(M, 1) * sizeof(ContactRec);
     }
     return hipSuccess;
 }
 
 hipError_t World::upload_mask(const uint8_t* mask, uint8_t** d_out) {
     if (!mask) { *d_out = nullptr; return hipSuccess; }
-    if (!d_mask) ZA_TRY(dalloc(this, &d_mask, E));
+    if (!d_mask) ZA_TRY(grow(&d_mask, E));
     ZA_TRY(hipStreamSynchronize(stream));  // h_mask_stage may still feed an earlier copy
     std::memcpy(h_mask_stage, mask, E);
     ZA_TRY(hipMemcpyAsync(d_mask, h_mask_stage, E, hipMemcpyHostToDevice, stream));
@@ -810,7 +888,7 @@ hipError_t World::write_state_array(float4* dst, MirrorId mid, const float* src,
         ZA_TRY(hipStreamSynchronize(stream));
         ZA_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
     } else {
-        if (!d_stage) ZA_TRY(dalloc(this, &d_stage, (size_t)E * B));
+        if (!d_stage) ZA_TRY(grow(&d_stage, (size_t)E * B));
         uint8_t* dm = nullptr;
         ZA_TRY(upload_mask(mask, &dm));
         ZA_TRY(hipMemcpyAsync(d_stage, src, bytes, hipMemcpyHostToDevice, stream));
