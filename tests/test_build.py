@@ -34,6 +34,14 @@ def test_one_environment_shapes_keep_two_waves_per_simd():
 
 
 @pytest.mark.skipif(not Path(RESOURCES).exists(), reason="library not built here")
+def test_one_environment_lds_shapes_keep_three_waves_per_simd():
+    """The one-environment shapes whose contact list is in HBM run three waves per SIMD, on which
+    the number of environments they keep resident rests."""
+    occ = step_occupancy(Path(RESOURCES).read_text())
+    assert all(occ.get(shape, 0) >= 3 for shape in ("1,1,0", "1,1,0,grouped", "1,0,0", "1,0,0,grouped", "1,0,0,split")), occ
+
+
+@pytest.mark.skipif(not Path(RESOURCES).exists(), reason="library not built here")
 def test_grouped_instances_keep_the_occupancy_of_their_shape():
     """The extended-contact instances (narrow phase grouped by geom-type pair) launch where
     the placement choice scored the ungrouped shape, so they must fit as many waves."""

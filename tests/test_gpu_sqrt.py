@@ -1,10 +1,9 @@
 """The joint and contact solves take the square roots they compare against a threshold (C > 1e-6,
-sin > 1e-6, tangent speed > 1e-6, quaternion length > 1e-8) with `sqrt_gate` (dmath.h):
-v_sqrt_f32 and the one-ulp correction of a correctly rounded fp32 root, without the scaling of
-inputs below 2^-96. The same device code, through zeno_amd_selfcheck_sqrt, against numpy's IEEE
-fp32 square root: every significand of twelve binades (even and odd exponents, both ends of the
-range, the 2^-96 boundary), random bit patterns over the whole range, and the special values;
-below 2^-96 the result must stay under 2^-47, below every threshold it is compared with."""
+sin > 1e-6, tangent speed > 1e-6, quaternion length > 1e-8) with `sqrt_gate` (dmath.h): v_sqrt_f32
+and one Newton step on its exact residual with v_rsq_f32. The same device code, through
+zeno_amd_selfcheck_sqrt, against numpy's IEEE fp32 square root: every value from 2^-96 up, random
+bit patterns over the whole range, and the special values; below 2^-96 the result must stay under
+2^-47, below every threshold it is compared with."""
 import ctypes as C
 
 import numpy as np
@@ -43,6 +42,13 @@ def test_every_significand_of_a_binade(e):
     bits = np.arange(2**23, dtype=np.uint32) | np.uint32((e + 127) << 23)
     x = bits.view(np.float32)
     assert_same_bits(device_roots(x), ieee_roots(x), f"binade 2^{e}")
+
+
+@pytest.mark.parametrize("first", range(-96, 128, 16))
+def test_every_value_of_sixteen_binades(first):
+    for e in range(first, first + 16):
+        x = (np.arange(2**23, dtype=np.uint32) | np.uint32((e + 127) << 23)).view(np.float32)
+        assert_same_bits(device_roots(x), np.sqrt(x), f"binade 2^{e}")
 
 
 def test_random_bit_patterns():
