@@ -28,18 +28,23 @@ def test_workgroups_that_the_lds_holds(tmp_path):
 
 
 def test_smallest_pool(tmp_path):
-    """(bodies, free bodies, list) -> slots: robots by their bodies, piles by how many copies of a
-    body's ground contact their list holds, never below the most valid slots seen settled (the last
-    number, with the list's own length as the bound)."""
-    seen = [(13, 12, 64, 22), (13, 12, 128, 21), (25, 24, 64, 59), (25, 24, 80, 58), (25, 24, 128, 33), (25, 24, 200, 24),
-            (39, 38, 64, 62), (39, 38, 80, 76), (39, 38, 128, 90), (39, 38, 200, 56), (39, 38, 256, 35), (41, 40, 200, 48),
-            (51, 50, 128, 100), (51, 50, 200, 96), (51, 50, 256, 68), (51, 50, 384, 26), (63, 62, 128, 108), (63, 62, 200, 115),
-            (63, 62, 256, 120), (63, 62, 384, 69), (63, 62, 512, 30)]
-    rows = run(tmp_path, "\n".join(f'printf("%u\\n", pool_floor({b}, {n}, {m}));' for b, n, m, _ in seen)
-               + 'printf("%u %u %u\\n", pool_floor(14, 0, 64), pool_floor(30, 0, 64), pool_floor(2, 0, 1));')
-    for (b, n, m, most), (slots,) in zip(seen, rows):
-        assert min(slots, m) >= most, (b, n, m, slots, most)
-    assert rows[-1] == [24, 32, 24]
+    """Robots by their bodies, piles by how many copies of a body's ground contact their list holds:
+    (free bodies, list, most valid slots seen settled) in the extended mode, never below the last
+    number with the list's own length as the bound; (free, round, list, valid slots of 99 in a hundred
+    environments) in the reference's mode."""
+    extended = [(12, 64, 22), (12, 128, 21), (24, 64, 59), (24, 80, 58), (24, 128, 33), (24, 200, 24), (38, 64, 62), (38, 80, 76),
+                (38, 128, 90), (38, 200, 56), (38, 256, 35), (50, 128, 100), (50, 200, 96), (50, 256, 68), (50, 384, 26),
+                (62, 128, 108), (62, 200, 115), (62, 256, 120), (62, 384, 69), (62, 512, 30)]
+    plain = [(12, 8, 64, 12), (24, 16, 64, 36), (40, 27, 64, 40), (50, 34, 64, 37), (64, 43, 64, 43), (64, 43, 128, 71), (40, 27, 200, 36)]
+    rows = run(tmp_path, "\n".join([f'printf("%u\\n", pool_floor(0, {n}, {n}, {m}, true));' for n, m, _ in extended]
+                                   + [f'printf("%u\\n", pool_floor(0, {n}, {r}, {m}, false));' for n, r, m, _ in plain])
+               + 'for (bool e : {false, true}) printf("%u %u %u %u\\n", pool_floor(13, 0, 0, 64, e), pool_floor(29, 0, 0, 64, e),'
+                 ' pool_floor(1, 0, 0, 1, e), pool_floor(13, 2, 2, 64, e));')
+    for (n, m, most), (slots,) in zip(extended, rows):
+        assert min(slots, m) >= most, (n, m, slots, most)
+    for (n, r, m, most), (slots,) in zip(plain, rows[len(extended):]):
+        assert min(slots, m) >= most, (n, r, m, slots, most)
+    assert rows[-2:] == [[24, 32, 24, 24]] * 2
 
 
 def test_steps_of_a_captured_launch(tmp_path):

@@ -190,11 +190,15 @@ inline size_t lds_workgroups(size_t bytes) { return bytes == 0 ? kLdsPerCu : kLd
 // filled), then the levels.
 constexpr uint32_t kPoolMaxList = 1536;  // longer lists keep placement 3 (everything in HBM), as documented
 constexpr uint32_t kPoolFloor = 24;    // smallest pool offered (or the list, or one slot per body)
-// Smallest pool offered for lists of M slots: of B bodies, n_free hang on no joint (World::pool_sizes).
-inline uint32_t pool_floor(uint32_t B, uint32_t n_free, uint32_t M) {
-    const uint64_t n = n_free, half_slots = M < 5 * n ? 5 * n : M < 7 * n ? 3 * n : 2 * n;
-    const uint64_t slots = std::max<uint64_t>((half_slots + 1) / 2, B);
-    return (uint32_t)std::max<uint64_t>(kPoolFloor, (slots + 7) / 8 * 8);
+// Smallest pool offered for lists of M slots (World::pool_sizes): `held` moving bodies hang on joints,
+// n_free do not, and n_round of those have a sphere or capsule, the shapes that meet the ground in the
+// reference's contact mode.
+inline uint32_t pool_floor(uint32_t held, uint32_t n_free, uint32_t n_round, uint32_t M, bool extended) {
+    const uint64_t n = n_free;
+    uint64_t slots;
+    if (extended) slots = M < 5 * n ? (5 * n + 1) / 2 : M < 7 * n ? (3 * n + 1) / 2 : n;
+    else slots = M < 3 * n ? (uint64_t)(M / n_free) * n_round + std::min(n_round, M % n_free) : M < 7 * n ? (3 * n + 1) / 2 : n;
+    return (uint32_t)std::max<uint64_t>(kPoolFloor, (held + slots + 3) / 4 * 4);
 }
 constexpr uint32_t kBodyQuadsSplit = 9, kBodyQuads = 7;
 constexpr uint32_t kPoolClasses = 64;  // ordered geom-type pairs of the grouped narrow phase

@@ -655,10 +655,15 @@ hipError_t World::step(const float* actions, uint32_t substeps, bool actions_on_
 // steps; 24 slots or the whole list take the same time within 3%, and a pool of one slot, where
 // every contact overflows, 4-15% more): kPoolFloor or a slot per body.
 // A free body can lie on the ground with as many valid slots as the list holds copies of its plane
-// pair. Settled piles of 12 to 62 bodies have had at most 2.4 valid slots per body where the list
-// holds fewer than five per body, 1.5 below seven (38 bodies and 200 slots: 148 us with 40 slots,
-// 118 with 64) and 1 above, where so many copies throw the bodies off the ground; only 12 bodies in
-// lists of 200 and more passed that, in one environment of a hundred at most.
+// pair. In the reference's contact mode spheres and capsules alone do: with fewer than three copies
+// the pool holds them all (64 bodies, a third of them boxes: 43 of 64 slots), with up to seven 1.5 per
+// body, above 1, as so many copies throw the bodies off the ground (40 bodies and 200 slots: 251 us
+// with the whole list, 153 with 64 slots; 20 bodies, 64 slots, 4600 environments: 355 us with 56, where
+// two rounds are needed, 282 with 24). In the extended mode settled piles of 12 to 62 bodies have had
+// at most 2.4 valid slots per body where the list holds fewer than five copies, 1.5 below seven (38
+// bodies and 200 slots: 148 us with 40 slots, 118 with 64) and 1 above; only 12 bodies in lists of 200
+// and more passed that, in one environment of a hundred at most. Lists of fewer than 64 slots keep
+// their shape when the mode is switched on, so they have its floor from the start.
 // ZENO_AMD_POOL=n (tests of pools that overflow) offers n alone.
 std::vector<uint32_t> World::pool_sizes() const {
     const uint32_t m = std::max<uint32_t>(M, 1);
@@ -666,11 +671,17 @@ std::vector<uint32_t> World::pool_sizes() const {
         const int n = std::atoi(env);
         if (n > 0) return {std::min((uint32_t)n, m)};
     }
-    std::vector<uint8_t> free_body(B, 1);
-    for (const ConstraintRec& c : model.templates) free_body[c.indices[0]] = free_body[c.indices[1]] = 0;
-    uint32_t n_free = 0;
-    for (uint32_t b = 0; b < B; ++b) n_free += free_body[b] && model.inv_mass_inertia[4 * b] > 0.0f ? 1u : 0u;
-    const uint32_t floor = std::min(m, pool_floor(B, n_free, M));
+    std::vector<uint8_t> on_joint(B, 0), round(B, 0);
+    for (const ConstraintRec& c : model.templates) on_joint[c.indices[0]] = on_joint[c.indices[1]] = 1;
+    for (const GeomRec& g : model.geoms) round[g.type_body[1]] |= g.type_body[0] == GEOM_SPHERE || g.type_body[0] == GEOM_CAPSULE ? 1 : 0;
+    uint32_t held = 0, n_free = 0, n_round = 0;
+    for (uint32_t b = 0; b < B; ++b) {
+        if (!(model.inv_mass_inertia[4 * b] > 0.0f)) continue;
+        if (on_joint[b]) { ++held; continue; }
+        ++n_free;
+        n_round += round[b];
+    }
+    const uint32_t floor = std::min(m, pool_floor(held, n_free, n_round, M, ext_contacts || M < 64u));
     std::vector<uint32_t> sizes{m};
     for (uint32_t c : {512u, 256u, 192u, 128u, 96u, 64u, 48u, 32u, 24u}) {
         if (c < m && c >= floor) sizes.push_back(c);
@@ -682,7 +693,7 @@ std::vector<uint32_t> World::pool_sizes() const {
 void World::set_extended_contacts(bool on) {
     release_graph();
     ext_contacts = on;
-    if (shape_forced || base_placement != PL_LDS || hash) return;
+    if (shape_forced || base_placement > PL_MODEL_HBM || hash) return;
     placement = base_placement;
     epw = base_epw;
     waves = base_waves;
@@ -713,8 +724,10 @@ void World::set_extended_contacts(bool on) {
             lds = l;
         }
     };
-    for (int w : {4, 1, 2}) {
-        for (uint32_t cap : pool_sizes()) offer(PL_LDS, w, cap);
+    if (base_placement == PL_LDS) {
+        for (int w : {4, 1, 2}) {
+            for (uint32_t cap : pool_sizes()) offer(PL_LDS, w, cap);
+        }
     }
     for (uint32_t cap : pool_sizes()) offer(PL_MODEL_HBM, 1, cap);
 }
