@@ -127,3 +127,22 @@ def test_hits_of_negative_penetration(M):
         seen += int(((pen < 0) & (pen != -1)).sum())
         compare(gpu_arrays(g), oracle_arrays(o), 0.0, 0.0)
     assert seen > 0
+
+
+def test_extended_mode_takes_its_own_pool_with_records_in_hbm():
+    """Boxes meet the ground in the extended mode alone, so its pool is larger; a world whose model
+    records are in HBM switches to it and back."""
+    from zeno_amd.scenes import pile_mjcf
+    from zeno_amd.world import ZenoWorld
+
+    w = ZenoWorld(mjcf_string=pile_mjcf(64, seed=3), num_envs=6000, max_contacts_per_env=128)
+    base = (w.modes()["placement"], w.launch_config())
+    assert base[0] == 1
+    w.set_extended_contacts(True)
+    assert w.modes()["placement"] == 1 and w.launch_config()[1] > base[1][1]
+    for _ in range(3):
+        w.step(np.zeros((6000, 0), np.float32))
+    assert np.isfinite(w.get_body_positions()).all()
+    w.set_extended_contacts(False)
+    assert (w.modes()["placement"], w.launch_config()) == base
+    w.close()
